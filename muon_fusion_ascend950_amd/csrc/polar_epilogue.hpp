@@ -32,8 +32,8 @@ __device__ __forceinline__ u32x2 pack4(const uint16_t (&h)[4]) {
 }
 
 // Epilogue values of one output row-block i: 4 consecutive columns per (j, q).
-template <Stage S>
-__device__ __forceinline__ void epilogue_values(const f32x16 &acc, int q, const float (&e)[4],
+template <Stage S, class Acc>
+__device__ __forceinline__ void epilogue_values(const Acc &acc, int q, const float (&e)[4],
                                                 const GemmArgs &g, uint16_t (&h)[4]) {
     constexpr Stage E = StageTraits<S>::kEpilogue;
 #pragma unroll

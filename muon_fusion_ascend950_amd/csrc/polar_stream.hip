@@ -35,6 +35,7 @@
 #include "polar_tile.hpp"
 
 #include <type_traits>
+#include <utility>
 
 namespace muon_polar {
 
@@ -65,14 +66,33 @@ struct StreamGeom {
     // into the first slot the K loop stops refilling, so its latency overlaps the
     // last K-steps instead of following them.
     static constexpr bool kEpiInSlot = kTileBytes <= kStageBytes && D >= 3;
+    // Wave pairs (see stream_segment) and the 256x256 tiles with 8 waves, whose ring holds
+    // five 32 KiB panels (all of the LDS) instead of K-step slots.
+    static constexpr bool kPair = NW == 8 && ((BM == 192 && BN == 192) || (BM == 256 && BN == 128));
+    static constexpr bool kPanelRing = BM == 256 && BN == 256 && NW == 8;
+    static constexpr int kRingBytes = kPanelRing ? 5 * kABytes : D * kStageBytes;
+    // 1 KiB per wave past the ring that idle DMA instructions write, where a ring slot may
+    // hold the epilogue tile meanwhile (kEpiInSlot) or for the kernels they share code with.
+    static constexpr int kSinkBytes = kPair || kPanelRing ? 0 : NW * 1024;
     static_assert(D >= 2 && D <= 8, "ring depth");
     static_assert((D - 1) * kLoads + kEpiLoads <= 63, "vmcnt range");
     static_assert(kLoadsA >= 1 && kLoadsB >= 1 && kABytes % (1024 * NW) == 0 &&
                       kBBytes % (1024 * NW) == 0,
                   "panels must split into whole 1 KiB DMA blocks per wave");
-    static_assert(kTileBytes <= kStages * kStageBytes, "epilogue tile must fit the ring");
+    static_assert(kTileBytes <= kRingBytes - (kPanelRing ? 16 : 0),
+                  "epilogue tile must fit the ring");
     static_assert(kTileBytes % (1024 * NW) == 0, "epilogue DMA is whole 1 KiB blocks per wave");
 };
+
+// f(0), f(1), ..., f(N - 1) with the index a compile-time constant.
+template <class F, int... I>
+__device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+    static_for_seq(f, std::make_integer_sequence<int, N>{});
+}
 
 // s_waitcnt vmcnt(n * LOADS), workgroup barrier; n < NMAX known only at run time.
 template <int LOADS, int NMAX, int EXTRA = 0>
@@ -122,14 +142,13 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     // Wave pairs (8 waves on a 192x192 tile, whose 2 x 4 wave grid would not be
     // made of 32-wide MFMA blocks, or on a 256x128 apply tile, whose 2 x 4 grid
     // would read 5 fragments per 4 MFMAs): the tile is four wave tiles (96x96,
-    // 128x64), each computed by two waves — wave w and w + 4 — that split every
-    // K-step's four k16 slices between them (slices h and h + 2 for h = w / 4).
-    // Each wave pair reads each fragment once, as one wave of a 4-wave kernel
-    // does, and the two waves cover each other's LDS and barrier waits.  The
-    // halves are added once after the K loop (acc(h = 0) + acc(h = 1)), so each
-    // output sums its K terms in two interleaved chains: results differ in
-    // rounding from the single-chain kernels.
-    constexpr bool kPair = NW == 8 && ((BM == 192 && BN == 192) || (BM == 256 && BN == 128));
+    // 128x64), each computed by two waves — wave w and w + 4 — that take one k32
+    // slice of every K-step each (slice h = w / 4).  Each wave pair reads each
+    // fragment once, as one wave of a 4-wave kernel does, and the two waves cover
+    // each other's LDS and barrier waits.  The halves are added once after the K
+    // loop (acc(h = 0) + acc(h = 1)), so each output sums its K terms in two
+    // interleaved chains: results differ in rounding from the single-chain kernels.
+    constexpr bool kPair = Geo::kPair;
     constexpr int kGridWaves = kPair ? 4 : NW;
     // Diagonal pairs (DG, 64x64 tiles with 4 waves): waves 0-1 compute diagonal
     // tile 2p from the row panel, waves 2-3 tile 2p + 1 from the column panel.
@@ -144,7 +163,21 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     static_assert(!DG || (StageTraits<S>::kSymmetric && BM == 64 && BN == 64 && NW == 4),
                   "diagonal pairs: 64x64 tiles of a triangular stage, 4 waves");
     constexpr int WM = BM / 2, WN = DG ? BN : BN / (kGridWaves / 2);
-    constexpr int SM = WM / 32, SN = WN / 32;
+    constexpr bool kPanelRing = Geo::kPanelRing;
+    constexpr int kPanels = 5;
+    // MFMA shape: 16x16x32 in the large-tile kernels (256x256 with 8 waves, the wave
+    // pairs), else 32x32x16.  The large tiles run at the power limit (the clock falls as
+    // the MFMA pipe fills), and 16x16x32 takes less power per FLOP: a loop of MFMAs alone
+    // on random operands sustains 2069 against 1819 TFLOP/s, with the fragment reads of
+    // 128x64 wave tiles 1739 against 1617.  Same bits (mfma_16x16x32).  With the even DMA
+    // spacing below: [4096,14336] gram 207.7 -> 185.1 us, poly 72.0 -> 65.6, apply 393.1
+    // -> 351.3; [4,4096,4096] 257.8 -> 233.9, 266.8 -> 241.7, 451.3 -> 409.2.
+    // kB: the MFMA's rows and columns; kNQ: groups of 4 consecutive columns a lane holds
+    // of one block.
+    constexpr bool k16 = kPair || kPanelRing;
+    constexpr int kB = k16 ? 16 : 32, kNQ = k16 ? 1 : 4;
+    using AccT = std::conditional_t<k16, f32x4, f32x16>;
+    constexpr int SM = WM / kB, SN = WN / kB;
     constexpr int kMfmaPerSlice = SM * SN;
     // Threads that hold accumulators (the h = 0 waves in pair mode).
     constexpr int kAccThreads = kPair ? kThreads / 2 : kThreads;
@@ -191,6 +224,20 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     int tid = static_cast<int>(threadIdx.x);
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63;
+    // Row and first column, within the wave tile, of this lane's group q of block (i, j)
+    auto grp_r = [&](int i) { return i * kB + (lane & (kB - 1)); };
+    auto grp_c = [&](int j, int q) {
+        return k16 ? 16 * j + 4 * (lane >> 4) : 32 * j + 8 * q + 4 * (lane >> 5);
+    };
+    // Swizzles of the K- and N-contiguous panels
+    auto kcs = [&](int row) { return k16 ? kc_swz16(row) : kc_swz(row); };
+    auto ncs = [&](auto bn_c, int krow) {
+        constexpr int kN = decltype(bn_c)::value;
+        if constexpr (k16)
+            return nc_swz16<kN>(krow);
+        else
+            return nc_swz<kN>(krow);
+    };
 
     const int tlin = tile_base + lt;
     const int bt = tlin / g.tiles_per_batch;
@@ -211,7 +258,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     // instruction + lane, row-major) is K-row q / (rows / 8), position q % (rows / 8).
     constexpr int kAChunksPerKRow = BM / 8, kBChunksPerKRow = BN / 8;
     auto a_row = [&](int i) { return 8 * (wave * Geo::kLoadsA + i) + (lane >> 3); };
-    auto a_chunk = [&](int i) { return (lane & 7) ^ kc_swz(a_row(i)); };
+    auto a_chunk = [&](int i) { return (lane & 7) ^ kcs(a_row(i)); };
     auto a_krow = [&](int i) {  // N-contiguous row operand
         return ((wave * Geo::kLoadsA + i) * 64 + lane) / kAChunksPerKRow;
     };
@@ -221,14 +268,14 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     };
     auto b_kpos = [&](int i) { return ((wave * Geo::kLoadsB + i) * 64 + lane) % kBChunksPerKRow; };
     auto b_row = [&](int i) { return 8 * (wave * Geo::kLoadsB + i) + (lane >> 3); };
-    auto b_chunk = [&](int i) { return (lane & 7) ^ kc_swz(b_row(i)); };
+    auto b_chunk = [&](int i) { return (lane & 7) ^ kcs(b_row(i)); };
 
     uint32_t off_a[Geo::kLoadsA], off_b[Geo::kLoadsB];
 #pragma unroll
     for (int i = 0; i < Geo::kLoadsA; ++i) {
         if constexpr (Tr::kRowNC) {
             const int krow = a_krow(i);
-            const int c = a_kpos(i) ^ nc_swz<BM>(krow);
+            const int c = a_kpos(i) ^ ncs(std::integral_constant<int, BM>{}, krow);
             const int col = row0 + 8 * c;
             off_a[i] =
                 col < g.row_rows ? static_cast<uint32_t>((krow * g.ld_row + col) * 2) : kOob;
@@ -243,7 +290,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     for (int i = 0; i < Geo::kLoadsB; ++i) {
         if constexpr (Tr::kColNC) {
             const int krow = b_krow(i);
-            const int c = b_kpos(i) ^ nc_swz<BN>(krow);
+            const int c = b_kpos(i) ^ ncs(std::integral_constant<int, BN>{}, krow);
             const int col = col0 + 8 * c;
             off_b[i] =
                 col < g.col_rows ? static_cast<uint32_t>((krow * g.ld_col + col) * 2) : kOob;
@@ -255,13 +302,9 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
         }
     }
 
-    auto a_dst = [&](int slot, int i) {
-        return smem_base + slot * Geo::kStageBytes + (wave * Geo::kLoadsA + i) * 1024;
-    };
-    auto b_dst = [&](int slot, int i) {
-        return smem_base + slot * Geo::kStageBytes + Geo::kABytes +
-               (wave * Geo::kLoadsB + i) * 1024;
-    };
+    // LDS byte offsets of the panels in ring slot `slot`
+    auto slot_a = [&](int slot) { return slot * Geo::kStageBytes; };
+    auto slot_b = [&](int slot) { return slot * Geo::kStageBytes + Geo::kABytes; };
     auto a_step = [&](int k0) -> uint32_t {
         return static_cast<uint32_t>((Tr::kRowNC ? k0 * g.ld_row : k0) * 2);
     };
@@ -284,19 +327,28 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     // they read the zeros a padded copy of X would hold there, and the sums are
     // the padded copy's bit for bit.
     static_assert(!KT || (!Tr::kRowNC && !Tr::kColNC), "K masks of K-contiguous panels");
-    auto dma_one = [&](int d, int step, int slot, bool live) {
+    auto a_voff = [&](int d, int step, bool live) -> uint32_t {
         const int k0 = step * kBK;
+        const uint32_t koff = live ? a_step(k0) : kOob;
+        const uint32_t off = off_a[d] + koff;
+        if constexpr (KT) return k0 + 8 * a_chunk(d) < g.row_k ? off : kOob;
+        return off;
+    };
+    auto b_voff = [&](int i, int step, bool live) -> uint32_t {
+        const int k0 = step * kBK;
+        const uint32_t koff = live ? b_step(k0) : kOob;
+        const uint32_t off = off_b[i] + koff;
+        if constexpr (KT) return k0 + 8 * b_chunk(i) < g.col_k ? off : kOob;
+        return off;
+    };
+    auto dma_one = [&](int d, int step, int slot, bool live) {
         if (d < Geo::kLoadsA) {
-            const uint32_t koff = live ? a_step(k0) : kOob;
-            uint32_t off = off_a[d] + koff;
-            if constexpr (KT) off = k0 + 8 * a_chunk(d) < g.row_k ? off : kOob;
-            dma_16B(rs_row, live ? a_dst(slot, d) : sink_base, off);
+            const uint32_t dst = smem_base + slot_a(slot) + (wave * Geo::kLoadsA + d) * 1024;
+            dma_16B(rs_row, live ? dst : sink_base, a_voff(d, step, live));
         } else {
             const int i = d - Geo::kLoadsA;
-            const uint32_t koff = live ? b_step(k0) : kOob;
-            uint32_t off = off_b[i] + koff;
-            if constexpr (KT) off = k0 + 8 * b_chunk(i) < g.col_k ? off : kOob;
-            dma_16B(rs_col, live ? b_dst(slot, i) : sink_base, off);
+            const uint32_t dst = smem_base + slot_b(slot) + (wave * Geo::kLoadsB + i) * 1024;
+            dma_16B(rs_col, live ? dst : sink_base, b_voff(i, step, live));
         }
     };
     // KT with rows of n % 8 != 0 elements (gram reading X rows of even length in
@@ -321,23 +373,22 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
             }
         }
     }
-    auto fix_tail = [&](int slot_) {
+    auto fix_tail = [&](int ao, int bo) {
         if constexpr (KT == 2) {
             // an opaque copy of the wave index keeps this address arithmetic here
             // rather than hoisted out of the K loop (where its values would stay
             // live in scalar registers and spill)
             int wv = wave;
             asm volatile("" : "+s"(wv));
-            const uint32_t base = smem_base + slot_ * Geo::kStageBytes + 16 * lane;
 #pragma unroll
             for (int d = 0; d < Geo::kLoads; ++d) {
-                const uint32_t dst =
-                    d < Geo::kLoadsA
-                        ? base + (wv * Geo::kLoadsA + d) * 1024
-                        : base + Geo::kABytes + (wv * Geo::kLoadsB + d - Geo::kLoadsA) * 1024;
+                const int dst = (d < Geo::kLoadsA
+                                     ? ao + (wv * Geo::kLoadsA + d) * 1024
+                                     : bo + (wv * Geo::kLoadsB + d - Geo::kLoadsA) * 1024) +
+                                16 * lane;
                 // keep values 0 .. rem-1 of the chunk (all of it when rem is 0)
                 const int rem = static_cast<int>((tail_rem >> (4 * d)) & 15u);
-                u32x4 *q = reinterpret_cast<u32x4 *>(smem + (dst - smem_base) / 2);
+                u32x4 *q = reinterpret_cast<u32x4 *>(smem + dst / 2);
                 u32x4 v = *q;
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
@@ -385,21 +436,57 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     };
 
     // -------------------------------------------------------- main loop
-    f32x16 acc[SM][SN];
+    AccT acc[SM][SN];
 #pragma unroll
     for (int i = 0; i < SM; ++i)
 #pragma unroll
         for (int j = 0; j < SN; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+            for (int e = 0; e < 4 * kNQ; ++e) acc[i][j][e] = 0.0f;
 
     // MFMA operand fragments of one k16 slice, double-buffered in registers.
-    // Fragment f of k16 slice kk from `slot`: f < SM row-operand fragment f,
-    // else column-operand fragment f - SM.
-    auto load_frag = [&](int slot, int kk, int f, bf16x8 (&fr)[SM], bf16x8 (&fc)[SN]) {
-        const uint16_t *as = smem + slot * (Geo::kStageBytes / 2);
-        const uint16_t *bs = as + Geo::kABytes / 2;
-        if (f < SM) {
+    // Fragment f of k16 slice kk of the panels at LDS byte offsets (ao, bo): f < SM
+    // row-operand fragment f, else column-operand fragment f - SM.
+    lds_u8 *const smem3 = reinterpret_cast<lds_u8 *>(smem_base);
+    const uint32_t kc_lane = k16 ? frag16_kc_lane(lane) : 0u;
+    uint32_t nc_swz_row = 0, nc_row_row = 0, nc_swz_col = 0, nc_row_col = 0;
+    if constexpr (k16 && Tr::kRowNC) {
+        nc_swz_row = frag16_nc_swz<BM>(lane);
+        nc_row_row = frag16_nc_row<BM>(lane);
+    }
+    if constexpr (k16 && Tr::kColNC) {
+        nc_swz_col = frag16_nc_swz<BN>(lane);
+        nc_row_col = frag16_nc_row<BN>(lane);
+    }
+    auto load_frag = [&](int ao, int bo, int kk, int f, bf16x8 (&fr)[SM], bf16x8 (&fc)[SN]) {
+        const uint16_t *as = smem + ao / 2;
+        const uint16_t *bs = smem + bo / 2;
+        if constexpr (k16) {  // kk: k32 slice
+            // (`lane` parts opaque here: their combinations with the fragment's uniform part
+            // would otherwise all be formed outside the K loop and spill)
+            if (f < SM) {
+                if constexpr (Tr::kRowNC) {
+                    uint32_t x = nc_swz_row;
+                    asm volatile("" : "+v"(x));
+                    fr[f] = frag16_nc_tr<BM>(smem3 + ((x ^ uint32_t(2 * (wr * WM + 16 * f))) +
+                                                      (nc_row_row + ao + 64 * BM * kk)));
+                } else {
+                    fr[f] = frag16_kc(smem3 + ((kc_lane ^ (64 * kk)) + (ao + 128 * wr * WM)) +
+                                      128 * 16 * f);
+                }
+            } else {
+                const int j = f - SM;
+                if constexpr (Tr::kColNC) {
+                    uint32_t x = nc_swz_col;
+                    asm volatile("" : "+v"(x));
+                    fc[j] = frag16_nc_tr<BN>(smem3 + ((x ^ uint32_t(2 * (wc * WN + 16 * j))) +
+                                                      (nc_row_col + bo + 64 * BN * kk)));
+                } else {
+                    fc[j] = frag16_kc(smem3 + ((kc_lane ^ (64 * kk)) + (bo + 128 * wc * WN)) +
+                                      128 * 16 * j);
+                }
+            }
+        } else if (f < SM) {
             if constexpr (Tr::kRowNC)
                 fr[f] = frag_nc_tr<BM>(as, wr * WM + f * 32 + ((lane >> 4) & 1) * 16, kk, lane);
             else
@@ -412,23 +499,31 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
                 fc[j] = frag_kc(bs, wc * WN + j * 32 + (lane & 31), kk, lane);
         }
     };
-    auto load_frags = [&](int slot, int kk, bf16x8 (&fr)[SM], bf16x8 (&fc)[SN]) {
+    auto load_frags = [&](int ao, int bo, int kk, bf16x8 (&fr)[SM], bf16x8 (&fc)[SN]) {
 #pragma unroll
-        for (int f = 0; f < SM + SN; ++f) load_frag(slot, kk, f, fr, fc);
+        for (int f = 0; f < SM + SN; ++f) load_frag(ao, bo, kk, f, fr, fc);
     };
-    // a·X into the accumulators from the panel of global K-step kg in `slot`,
+    // a·X into the accumulators from the panels of global K-step kg at (ao, bo),
     // when that step's 64 K-values are 64 of this tile's rows (apply: X rows;
     // the column panel [64][BN] holds X[k][col0 + c]) or columns (apply-right:
     // X columns; the row panel [BM][64] holds X[row0 + r][k]).  Each lane adds
     // the 4 consecutive values its accumulator elements 4q..4q+3 cover, once
     // per output element over the whole K loop.
-    auto add_ax = [&](int slot, int kg) {
+    auto add_ax = [&](int ao, int bo, int kg) {
         if constexpr (kAxInLoop) {
             if (!acc_owner) return;  // wave pairs: a·X goes into the h = 0 half once
-            const uint16_t *as = smem + slot * (Geo::kStageBytes / 2);
-            const uint16_t *bs = as + Geo::kABytes / 2;
+            // an opaque copy of the lane index keeps the address arithmetic in the few
+            // steps that use it (hoisted out of the K loop it would spill)
+            int ln = lane;
+            asm volatile("" : "+v"(ln));
+            const int lane_r = ln & (kB - 1);
+            auto lane_c = [&](int j, int q) {
+                return k16 ? 16 * j + 4 * (ln >> 4) : 32 * j + 8 * q + 4 * (ln >> 5);
+            };
+            const uint16_t *as = smem + ao / 2;
+            const uint16_t *bs = smem + bo / 2;
             const float a = g.s_epi;
-            auto fma4 = [&](f32x16 &acc_ij, int q, u32x2 v) {
+            auto fma4 = [&](AccT &acc_ij, int q, u32x2 v) {
                 float x[4];
                 unpack4(v, x);
 #pragma unroll
@@ -437,48 +532,66 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
             if constexpr (S == Stage::Apply) {
                 const int rel = kg * kBK - row0;  // tile row of the step's first K-row
                 if (rel < 0 || rel >= BM) return;
+                // row blocks that fit a K-step share one branch
+                constexpr int kGrp = WM >= kBK ? kBK / kB : 1;
 #pragma unroll
-                for (int i = 0; i < SM; ++i) {
-                    const int rb = wr * WM + 32 * i;
+                for (int i0 = 0; i0 < SM; i0 += kGrp) {
+                    const int rb = wr * WM + kB * i0;
                     if (rb < rel || rb >= rel + kBK) continue;
-                    const int kr = rb - rel + (lane & 31);
 #pragma unroll
-                    for (int j = 0; j < SN; ++j)
+                    for (int i = i0; i < i0 + kGrp; ++i) {
+                        const int kr = rb + kB * (i - i0) - rel + lane_r;
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const int c = wc * WN + 32 * j + 8 * q + 4 * (lane >> 5);
-                            fma4(acc[i][j], q,
-                                 *reinterpret_cast<const u32x2 *>(
-                                     bs + nc_offset<BN>(kr, c >> 3) + (c & 7)));
-                        }
+                        for (int j = 0; j < SN; ++j)
+#pragma unroll
+                            for (int q = 0; q < kNQ; ++q) {
+                                const int c = wc * WN + lane_c(j, q);
+                                const int pos =
+                                    (c >> 3) ^ ncs(std::integral_constant<int, BN>{}, kr);
+                                fma4(acc[i][j], q,
+                                     *reinterpret_cast<const u32x2 *>(bs + kr * BN + 8 * pos +
+                                                                      (c & 7)));
+                            }
+                    }
                 }
             } else {
                 const int rel = kg * kBK - col0;  // tile column of the step's first K
                 if (rel < 0 || rel >= BN) return;
+                constexpr int kGrp = WN >= kBK ? kBK / kB : 1;
 #pragma unroll
-                for (int j = 0; j < SN; ++j) {
-                    const int cb = wc * WN + 32 * j;
+                for (int j0 = 0; j0 < SN; j0 += kGrp) {
+                    const int cb = wc * WN + kB * j0;
                     if (cb < rel || cb >= rel + kBK) continue;
 #pragma unroll
-                    for (int i = 0; i < SM; ++i) {
-                        const int r = wr * WM + 32 * i + (lane & 31);
+                    for (int j = j0; j < j0 + kGrp; ++j) {
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const int kc = cb - rel + 8 * q + 4 * (lane >> 5);
-                            fma4(acc[i][j], q,
-                                 *reinterpret_cast<const u32x2 *>(
-                                     as + kc_offset(r, kc >> 3) + (kc & 7)));
+                        for (int i = 0; i < SM; ++i) {
+                            const int r = wr * WM + kB * i + lane_r;
+#pragma unroll
+                            for (int q = 0; q < kNQ; ++q) {
+                                const int kc = wc * WN + lane_c(j, q) - rel;
+                                fma4(acc[i][j], q,
+                                     *reinterpret_cast<const u32x2 *>(
+                                         as + r * kBK + (((kc >> 3) ^ kcs(r)) << 3) +
+                                         (kc & 7)));
+                            }
                         }
                     }
                 }
             }
         }
     };
+    auto mfma = [&](const bf16x8 &c, const bf16x8 &r, const AccT &a) -> AccT {
+        if constexpr (k16)
+            return mfma_16x16x32(c, r, a);
+        else
+            return mfma_32x32x16(c, r, a);
+    };
     auto mfmas = [&](const bf16x8 (&fr)[SM], const bf16x8 (&fc)[SN]) {
 #pragma unroll
         for (int i = 0; i < SM; ++i)
 #pragma unroll
-            for (int j = 0; j < SN; ++j) acc[i][j] = mfma_32x32x16(fc[j], fr[i], acc[i][j]);
+            for (int j = 0; j < SN; ++j) acc[i][j] = mfma(fc[j], fr[i], acc[i][j]);
     };
     // Last slice of a step: its MFMAs with the DMA of panel `step` interleaved,
     // about kLoads / kMfmaPerSlice instructions after each MFMA (into the sink
@@ -493,9 +606,9 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
 #pragma unroll
         for (int m = 0; m < kMfmaPerSlice; ++m) {
             const int i = m / SN, j = m % SN;
-            acc[i][j] = mfma_32x32x16(fc[j], fr[i], acc[i][j]);
+            acc[i][j] = mfma(fc[j], fr[i], acc[i][j]);
             __builtin_amdgcn_sched_barrier(0);
-            if (m < SM + SN) load_frag(nslot, nkk, m, nfr, nfc);
+            if (m < SM + SN) load_frag(slot_a(nslot), slot_b(nslot), nkk, m, nfr, nfc);
 #pragma unroll
             for (int d = m * Geo::kLoads / kMfmaPerSlice;
                  d < (m + 1) * Geo::kLoads / kMfmaPerSlice; ++d)
@@ -503,7 +616,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int f = kMfmaPerSlice; f < SM + SN; ++f) load_frag(nslot, nkk, f, nfr, nfc);
+        for (int f = kMfmaPerSlice; f < SM + SN; ++f) load_frag(slot_a(nslot), slot_b(nslot), nkk, f, nfr, nfc);
     };
     static_assert(kBK / 16 == 4, "schedule below is written for four k16 slices per step");
 
@@ -523,55 +636,182 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     // would overwrite an epilogue tile fetched into a ring slot during the loop.
     static_assert(!(kPair && kEpiPrefetch), "wave pairs cannot prefetch the epilogue tile");
     const int npro = nkl < kStages ? nkl : kStages;
-    for (int i = 0; i < npro; ++i) issue_all(kbeg + i, i);
     int epi_slot = 0;
-    if (tail_fix && nkl == 1) {  // the segment is the tile's last K-step alone
-        wait_vm<0>();
-        fix_tail(0);
-    }
-    if constexpr (kEpiPrefetch) {
-        if (nkl < kStages) {
-            epi_slot = nkl;  // a slot the K loop never fills
-            issue_epi(epi_slot);
-            wait_panels_barrier<Geo::kLoads, kStages, kEpiLoadsU>(npro - 1);
+    if constexpr (!k16) {
+        for (int i = 0; i < npro; ++i) issue_all(kbeg + i, i);
+        if (tail_fix && nkl == 1) {  // the segment is the tile's last K-step alone
+            wait_vm<0>();
+            fix_tail(slot_a(0), slot_b(0));
+        }
+        if constexpr (kEpiPrefetch) {
+            if (nkl < kStages) {
+                epi_slot = nkl;  // a slot the K loop never fills
+                issue_epi(epi_slot);
+                wait_panels_barrier<Geo::kLoads, kStages, kEpiLoadsU>(npro - 1);
+            } else {
+                epi_slot = (nkl - kStages) % kStages;
+                wait_panels_barrier<Geo::kLoads, kStages>(npro - 1);
+            }
         } else {
-            epi_slot = (nkl - kStages) % kStages;
             wait_panels_barrier<Geo::kLoads, kStages>(npro - 1);
         }
-    } else {
-        wait_panels_barrier<Geo::kLoads, kStages>(npro - 1);
     }
-    int slot = 0;
-    if constexpr (kPair) {
-        // This wave's k16 slices of every K-step: ka = h and kb = h + 2, in the
-        // 4-wave kernel's schedule with two slices per step:
-        //   frags(kb) | mfma(ka) | wait panel k+1, barrier | frags(next ka) |
-        //   mfma(kb) + DMA panel k+kStages -> slot
-        const int ka = kh, kb = kh + 2;
-        bf16x8 fr0[SM], fc0[SN], fr1[SM], fc1[SN];
-        load_frags(0, ka, fr0, fc0);
-        for (int k = 0; k < nkl; ++k) {
-            const int next = slot + 1 == kStages ? 0 : slot + 1;
-            if constexpr (kAxInLoop) add_ax(slot, kbeg + k);
-            load_frags(slot, kb, fr1, fc1);
-            mfmas(fr0, fc0);
-            for (int z = 0; z < kMfmaPerSlice; ++z) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            }
+    // One slice's MFMAs (row blocks outer), each followed by the fragment read that falls
+    // due (of k32 slice kk of the panels at (ao, bo), into nfr and nfc) and by after(m).
+    // The reads take the column fragments first, into registers of their own, then the row
+    // fragments in order, each about when an older row fragment has had its last use:
+    // about ten row fragments live instead of twice eight.
+    auto mfma_slice = [&](const bf16x8 (&fr)[SM], const bf16x8 (&fc)[SN], int ao, int bo, int kk,
+                          bf16x8 (&nfr)[SM], bf16x8 (&nfc)[SN], auto &&after) {
+        static_for<kMfmaPerSlice>([&](auto mc) {
+            constexpr int m = decltype(mc)::value, i = m / SN, j = m % SN;
+            constexpr int kReads = SM + SN, kSpan = kMfmaPerSlice - 4;
+            acc[i][j] = mfma(fc[j], fr[i], acc[i][j]);
             __builtin_amdgcn_sched_barrier(0);
-            // the waits of the schedule below (panel k+1; later DMA groups in flight)
-            const int after = (npro - k - 2 > 0 ? npro - k - 2 : 0) + (k < kStages - 2 ? k : kStages - 2);
+            static_for<kReads>([&](auto rc) {
+                constexpr int r = decltype(rc)::value, f = r < SN ? SM + r : r - SN;
+                if constexpr (r * kSpan / kReads == m) load_frag(ao, bo, kk, f, nfr, nfc);
+            });
+            after(mc);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    int slot = 0;
+    // Steps [ax0, ax1) of the segment add a·X (add_ax): loops of their own, so that the
+    // others hold MFMAs, fragment reads and DMA only.
+    constexpr int kAxSteps = (S == Stage::Apply ? BM : BN) / kBK;
+    const int ax_first = (S == Stage::Apply ? row0 : col0) / kBK - kbeg;
+    auto in_segment = [&](int k) { return k < 0 ? 0 : k < nkl ? k : nkl; };
+    const int ax0 = in_segment(ax_first), ax1 = in_segment(ax_first + kAxSteps);
+    if constexpr (kPanelRing) {
+        // Per K-step k (panels A_k, B_k), k32 slices s0 and s1:
+        //   mfma(s0) + frags(s1) | wait panels k+1, barrier | mfma(s1) + frags(next s0)
+        // The barrier frees A_k's and B_k's places: column panel B_{k+2} then row panel
+        // A_{k+3} stream into them, one DMA instruction every kGap MFMAs over slice s1 and
+        // the next step's s0.  Issued together behind the barrier, the 64 instructions of
+        // a step (16 clocks each in the CU's address unit, half of a step's MFMA time)
+        // queue up and hold the waves' MFMAs back: MFMA pipe busy 68% of apply's cycles at
+        // [4096,14336] with two 64 KiB slots, 78% spread.  The half step more than two
+        // slots hold gives the spread panels time to land (8 MFMAs apart: 351 us; 4: 359).
+        // Idle instructions past the segment's end write zeros to places nothing reads.
+        static_assert(Geo::kABytes == Geo::kBBytes, "panel ring");
+        constexpr int kL = Geo::kLoadsA, kP = Geo::kABytes, kM = kMfmaPerSlice;
+        constexpr int kGap = kM / kL;
+        static_assert((2 * kL - 1) * kGap < 2 * kM, "a group is issued before the next barrier");
+        const uint32_t wave_dst = smem_base + wave * kL * 1024;
+        auto wrap = [](int p) { return p >= kPanels ? p - kPanels : p; };
+        // DMA instruction due after MFMA q of a group: column panel of step sb into position
+        // pos_b, then row panel of step sb + 1 into position pos_a.
+        auto group_at = [&](auto qc, int sb, int pos_b, int pos_a) {
+            constexpr int q = decltype(qc)::value, j = q / kGap;
+            if constexpr (q % kGap == 0 && j < kL)
+                dma_16B_at<j * 1024>(rs_col, wave_dst + pos_b * kP, b_voff(j, sb, sb < kend));
+            else if constexpr (q % kGap == 0 && j < 2 * kL)
+                dma_16B_at<(j - kL) * 1024>(rs_row, wave_dst + pos_a * kP,
+                                            a_voff(j - kL, sb + 1, sb + 1 < kend));
+        };
+        static_for<kL>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            dma_16B_at<j * 1024>(rs_row, wave_dst, a_voff(j, kbeg, true));
+        });
+        static_for<kL>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            dma_16B_at<j * 1024>(rs_col, wave_dst + kP, b_voff(j, kbeg, true));
+        });
+        static_for<kL>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            dma_16B_at<j * 1024>(rs_row, wave_dst + 2 * kP, a_voff(j, kbeg + 1, 1 < nkl));
+        });
+        static_for<kM>([&](auto mc) { group_at(mc, kbeg + 1, 3, 4); });
+        if (tail_fix && nkl == 1) {  // the segment is the tile's last K-step alone
+            wait_vm<0>();
+            fix_tail(0, kP);
+        }
+        wait_vm_barrier<kL + (kM + kGap - 1) / kGap>();
+        bf16x8 fr0[SM], fc0[SN], fr1[SM], fc1[SN];
+        load_frags(0, kP, 0, fr0, fc0);
+        int pa = 0, k = 0;
+        auto step = [&](auto ax_c) {
+            const int pb = wrap(pa + 1), na = wrap(pa + 2), nb = wrap(pa + 3), pz = wrap(pa + 4);
+            if constexpr (decltype(ax_c)::value) add_ax(pa * kP, pb * kP, kbeg + k);
+            mfma_slice(fr0, fc0, pa * kP, pb * kP, 1, fr1, fc1, [&](auto mc) {
+                group_at(std::integral_constant<int, kM + decltype(mc)::value>{}, kbeg + k + 1,
+                         nb, pz);
+            });
             if (tail_fix && k == nkl - 2) {
                 wait_vm<0>();
-                fix_tail(next);
+                fix_tail(na * kP, nb * kP);
             }
-            wait_panels_barrier<Geo::kLoads, kStages - 1>(after);
-            mfmas_with_dma_frags(fr1, fc1, kbeg + k + kStages, slot, k + kStages < nkl, next, fr0,
-                                 fc0, ka);
-            __builtin_amdgcn_sched_barrier(0);
-            slot = next;
+            wait_vm_barrier<kL>();
+            mfma_slice(fr1, fc1, na * kP, nb * kP, 0, fr0, fc0,
+                       [&](auto mc) { group_at(mc, kbeg + k + 2, pa, pb); });
+            pa = na;
+            ++k;
+        };
+        if constexpr (kAxInLoop) {
+            while (k < ax0) step(std::false_type{});
+            while (k < ax1) step(std::true_type{});
         }
+        while (k < nkl) step(std::false_type{});
+    } else if constexpr (kPair) {
+        // This wave's k32 slice h of every K-step; per step k:
+        //   wait panel k+1, barrier | mfma + frags(k+1) + DMA panel k+kStages -> slot of k
+        // (its fragments of step k are in registers before the barrier).
+        constexpr int kM = kMfmaPerSlice, kL = Geo::kLoads, kGap = kM / kL;
+        const uint32_t dst_a = smem_base + wave * Geo::kLoadsA * 1024;
+        const uint32_t dst_b = smem_base + Geo::kABytes + wave * Geo::kLoadsB * 1024;
+        auto dma_c = [&](auto dc, int step, int sl) {
+            constexpr int d = decltype(dc)::value;
+            if constexpr (d < Geo::kLoadsA)
+                dma_16B_at<d * 1024>(rs_row, dst_a + sl * Geo::kStageBytes,
+                                     a_voff(d, step, step < kend));
+            else
+                dma_16B_at<(d - Geo::kLoadsA) * 1024>(
+                    rs_col, dst_b + sl * Geo::kStageBytes,
+                    b_voff(d - Geo::kLoadsA, step, step < kend));
+        };
+        for (int i = 0; i < kStages; ++i)
+            static_for<kL>([&](auto dc) { dma_c(dc, kbeg + i, i); });
+        if (tail_fix && nkl == 1) {
+            wait_vm<0>();
+            fix_tail(slot_a(0), slot_b(0));
+        }
+        wait_vm_barrier<(kStages - 1) * kL>();
+        bf16x8 fr0[SM], fc0[SN], fr1[SM], fc1[SN];
+        load_frags(slot_a(0), slot_b(0), kh, fr0, fc0);
+        int k = 0;
+        auto step = [&](auto ax_c, const bf16x8 (&fr)[SM], const bf16x8 (&fc)[SN],
+                        bf16x8 (&nfr)[SM], bf16x8 (&nfc)[SN]) {
+            const int next = slot + 1 == kStages ? 0 : slot + 1;
+            if constexpr (decltype(ax_c)::value) add_ax(slot_a(slot), slot_b(slot), kbeg + k);
+            if (tail_fix && k == nkl - 2) {
+                wait_vm<0>();
+                fix_tail(slot_a(next), slot_b(next));
+            }
+            wait_vm_barrier<(kStages - 2) * kL>();
+            mfma_slice(fr, fc, slot_a(next), slot_b(next), kh, nfr, nfc, [&](auto mc) {
+                constexpr int m = decltype(mc)::value;
+                if constexpr (m % kGap == 0 && m / kGap < kL)
+                    dma_c(std::integral_constant<int, m / kGap>{}, kbeg + k + kStages, slot);
+            });
+            slot = next;
+            ++k;
+        };
+        // pairs of steps up to `end` (even, or the segment's end)
+        auto steps = [&](auto ax_c, int end) {
+            while (k + 1 < end) {
+                step(ax_c, fr0, fc0, fr1, fc1);
+                step(ax_c, fr1, fc1, fr0, fc0);
+            }
+        };
+        if constexpr (kAxInLoop) {
+            // (whole tiles: kbeg = 0, and ax0 and ax1 are even but for the segment's end)
+            steps(std::false_type{}, ax0);
+            steps(std::true_type{}, ax1);
+            if (k < ax1) step(std::true_type{}, fr0, fc0, fr1, fc1);
+        }
+        steps(std::false_type{}, nkl);
+        if (k < nkl) step(std::false_type{}, fr0, fc0, fr1, fc1);
     } else if constexpr (DG) {
         // Fragments of one K-step, slices taken in the order s_i = (2h + i) mod 4:
         // o[i] = rows 32h.. (own block), t[i] = rows 32(1-h).. (shared block, i < 2).
@@ -598,7 +838,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
             const int after = (npro - k - 2 > 0 ? npro - k - 2 : 0) + (k < kStages - 2 ? k : kStages - 2);
             if (tail_fix && k == nkl - 2) {
                 wait_vm<0>();
-                fix_tail(next);
+                fix_tail(slot_a(next), slot_b(next));
             }
             if (kEpiPrefetch && k > nkl - kStages)
                 wait_panels_barrier<Geo::kLoads, kStages - 1, kEpiLoadsU>(after);
@@ -614,9 +854,9 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
                 // m = 0..5: own(0), shared(0), own(1), shared(1), own(2), own(3)
                 const int i = m < 4 ? m >> 1 : m - 2;
                 if (m < 4 && (m & 1))
-                    acc[0][1] = mfma_32x32x16(t[i & 1], o[i], acc[0][1]);
+                    acc[0][1] = mfma(t[i & 1], o[i], acc[0][1]);
                 else
-                    acc[0][0] = mfma_32x32x16(o[i], o[i], acc[0][0]);
+                    acc[0][0] = mfma(o[i], o[i], acc[0][0]);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int d = m * Geo::kLoads / kM; d < (m + 1) * Geo::kLoads / kM; ++d)
@@ -645,7 +885,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
         bf16x8 ar[4][SM], ac[4][SN], br[4][SM], bc[4][SN];
         auto read_step = [&](int sl, bf16x8 (&r)[4][SM], bf16x8 (&c)[4][SN]) {
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) load_frags(sl, kk, r[kk], c[kk]);
+            for (int kk = 0; kk < 4; ++kk) load_frags(slot_a(sl), slot_b(sl), kk, r[kk], c[kk]);
         };
         auto step = [&](int k, const bf16x8 (&r)[4][SM], const bf16x8 (&c)[4][SN],
                         bf16x8 (&nr)[4][SM], bf16x8 (&nc)[4][SN]) {
@@ -655,7 +895,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
             const int after = (npro - k - 2 > 0 ? npro - k - 2 : 0) + (k < kStages - 2 ? k : kStages - 2);
             if (tail_fix && k == nkl - 2) {
                 wait_vm<0>();
-                fix_tail(next);
+                fix_tail(slot_a(next), slot_b(next));
             }
             if (kEpiPrefetch && k > nkl - kStages)
                 wait_panels_barrier<Geo::kLoads, kStages - 1, kEpiLoadsU>(after);
@@ -670,7 +910,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
             for (int m = 0; m < kM; ++m) {
                 const int kk = m / kMfmaPerSlice, ij = m % kMfmaPerSlice;
                 acc[ij / SN][ij % SN] =
-                    mfma_32x32x16(c[kk][ij % SN], r[kk][ij / SN], acc[ij / SN][ij % SN]);
+                    mfma(c[kk][ij % SN], r[kk][ij / SN], acc[ij / SN][ij % SN]);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int d = m * Geo::kLoads / kM; d < (m + 1) * Geo::kLoads / kM; ++d)
@@ -678,14 +918,14 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
                 __builtin_amdgcn_sched_barrier(0);
             }
             if constexpr (kAxInLoop) {
-                if (k + 1 < nkl) add_ax(next, kbeg + k + 1);
+                if (k + 1 < nkl) add_ax(slot_a(next), slot_b(next), kbeg + k + 1);
             }
             if constexpr (kEpiPrefetch) {
                 if (k == nkl - kStages) issue_epi(epi_slot);
             }
             slot = next;
         };
-        if constexpr (kAxInLoop) add_ax(0, kbeg);
+        if constexpr (kAxInLoop) add_ax(slot_a(0), slot_b(0), kbeg);
         read_step(0, ar, ac);
         int k = 0;
         for (; k + 1 < nkl; k += 2) {
@@ -695,25 +935,25 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
         if (k < nkl) step(k, ar, ac, br, bc);
     } else {
         bf16x8 fr0[SM], fc0[SN], fr1[SM], fc1[SN];
-        load_frags(0, 0, fr0, fc0);
+        load_frags(slot_a(0), slot_b(0), 0, fr0, fc0);
         for (int k = 0; k < nkl; ++k) {
             const int next = slot + 1 == kStages ? 0 : slot + 1;
-            if constexpr (kAxInLoop) add_ax(slot, kbeg + k);
-            load_frags(slot, 1, fr1, fc1);
+            if constexpr (kAxInLoop) add_ax(slot_a(slot), slot_b(slot), kbeg + k);
+            load_frags(slot_a(slot), slot_b(slot), 1, fr1, fc1);
             mfmas(fr0, fc0);
             for (int z = 0; z < kMfmaPerSlice; ++z) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
-            load_frags(slot, 2, fr0, fc0);
+            load_frags(slot_a(slot), slot_b(slot), 2, fr0, fc0);
             mfmas(fr1, fc1);
             for (int z = 0; z < kMfmaPerSlice; ++z) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
-            load_frags(slot, 3, fr1, fc1);
+            load_frags(slot_a(slot), slot_b(slot), 3, fr1, fc1);
             mfmas(fr0, fc0);
             for (int z = 0; z < kMfmaPerSlice; ++z) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -732,7 +972,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
             const int after = (npro - k - 2 > 0 ? npro - k - 2 : 0) + (k < kStages - 2 ? k : kStages - 2);
             if (tail_fix && k == nkl - 2) {
                 wait_vm<0>();
-                fix_tail(next);
+                fix_tail(slot_a(next), slot_b(next));
             }
             if (kEpiPrefetch && k > nkl - kStages)
                 wait_panels_barrier<Geo::kLoads, kStages - 1, kEpiLoadsU>(after);
@@ -782,7 +1022,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     if constexpr (kPair) {
         constexpr int kF = SM * SN;
         constexpr int kF0 = (kF + 1) / 2;
-        static_assert(4 * kF0 * 4 * 64 * 16 <= kStages * Geo::kStageBytes,
+        static_assert(4 * kF0 * kNQ * 64 * 16 <= kStages * Geo::kStageBytes,
                       "pair reduction buffer must fit the ring");
         f32x4 *buf = reinterpret_cast<f32x4 *>(smem);
         auto round = [&](auto lo_c, auto hi_c) {
@@ -791,9 +1031,9 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
 #pragma unroll
                 for (int f = lo; f < hi; ++f)
 #pragma unroll
-                    for (int e4 = 0; e4 < 4; ++e4) {
-                        const f32x16 &a = acc[f / SN][f % SN];
-                        buf[((wq * kF0 + (f - lo)) * 4 + e4) * 64 + lane] =
+                    for (int e4 = 0; e4 < kNQ; ++e4) {
+                        const AccT &a = acc[f / SN][f % SN];
+                        buf[((wq * kF0 + (f - lo)) * kNQ + e4) * 64 + lane] =
                             f32x4{a[4 * e4], a[4 * e4 + 1], a[4 * e4 + 2], a[4 * e4 + 3]};
                     }
             }
@@ -802,9 +1042,9 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
 #pragma unroll
                 for (int f = lo; f < hi; ++f)
 #pragma unroll
-                    for (int e4 = 0; e4 < 4; ++e4) {
-                        const f32x4 v = buf[((wq * kF0 + (f - lo)) * 4 + e4) * 64 + lane];
-                        f32x16 &a = acc[f / SN][f % SN];
+                    for (int e4 = 0; e4 < kNQ; ++e4) {
+                        const f32x4 v = buf[((wq * kF0 + (f - lo)) * kNQ + e4) * 64 + lane];
+                        AccT &a = acc[f / SN][f % SN];
 #pragma unroll
                         for (int t = 0; t < 4; ++t) a[4 * e4 + t] = a[4 * e4 + t] + v[t];
                     }
@@ -842,7 +1082,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
         auto lane_base = [&](int u) {
             return static_cast<uint32_t>(int64_t(sk_slot(u, lt)) * slot_bytes) + tid * 16;
         };
-        // Slot layout: 16-byte chunk c = (i * SN + j) * 4 + q of every thread that
+        // Slot layout: 16-byte chunk c = (i * SN + j) * kNQ + q of every thread that
         // holds accumulators, thread-minor, so each access instruction covers 1 KiB
         // contiguously.
         constexpr uint32_t kChunkStride = kAccThreads * 16;
@@ -854,11 +1094,11 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
 #pragma unroll
                 for (int j = 0; j < SN; ++j)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
+                    for (int q = 0; q < kNQ; ++q)
                         __builtin_amdgcn_raw_buffer_store_b128(
                             f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
                                   acc[i][j][4 * q + 3]},
-                            rs_part, base + ((i * SN + j) * 4 + q) * kChunkStride, 0, kSc1);
+                            rs_part, base + ((i * SN + j) * kNQ + q) * kChunkStride, 0, kSc1);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         };
         if (tid == 0)
@@ -909,14 +1149,14 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
             // blocks of kBlk accumulator tiles (i, j), the next block's loads in
             // flight while one is added (one row-block of SN tiles; one tile
             // for the 256-register accumulators)
-            constexpr int kBlk = kBigAcc ? 1 : SN;
+            constexpr int kBlk = kBigAcc ? 1 : k16 ? (SM % 2 == 0 ? 2 * SN : SN) : SN;
             constexpr int kBlocks = SM * SN / kBlk;
-            f32x4 x[2][kBlk * 4];
-            auto load_block = [&](int blk, f32x4 (&dst)[kBlk * 4]) {
+            f32x4 x[2][kBlk * kNQ];
+            auto load_block = [&](int blk, f32x4 (&dst)[kBlk * kNQ]) {
 #pragma unroll
-                for (int c = 0; c < kBlk * 4; ++c)
+                for (int c = 0; c < kBlk * kNQ; ++c)
                     dst[c] = __builtin_amdgcn_raw_buffer_load_b128(
-                        rs_part, base + (blk * kBlk * 4 + c) * kChunkStride, 0, kSc1);
+                        rs_part, base + (blk * kBlk * kNQ + c) * kChunkStride, 0, kSc1);
             };
             load_block(0, x[0]);
 #pragma unroll
@@ -926,12 +1166,12 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
                 for (int t = 0; t < kBlk; ++t) {
                     const int ij = blk * kBlk + t, i = ij / SN, j = ij % SN;
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
+                    for (int q = 0; q < kNQ; ++q)
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            acc[i][j][4 * q + e] = assign ? x[blk & 1][t * 4 + q][e]
+                            acc[i][j][4 * q + e] = assign ? x[blk & 1][t * kNQ + q][e]
                                                           : acc[i][j][4 * q + e] +
-                                                                x[blk & 1][t * 4 + q][e];
+                                                                x[blk & 1][t * kNQ + q][e];
                 }
             }
         };
@@ -962,15 +1202,15 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     if (acc_owner) {
 #pragma unroll
         for (int i = 0; i < SM; ++i) {
-            const int r = wr * WM + i * 32 + (lane & 31);
+            const int r = wr * WM + grp_r(i);
 #pragma unroll
             for (int j = 0; j < SN; ++j) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
+                for (int q = 0; q < kNQ; ++q) {
                     // diagonal pairs: block (h,h), and (0,1) for h = 0
                     if (DG && hr == 1 && j == 1) continue;
-                    const int cb = DG ? (j == 0 ? 32 * hr : 32) : wc * WN + j * 32;
-                    const int c = cb + 8 * q + 4 * (lane >> 5);
+                    const int c = DG ? (j == 0 ? 32 * hr : 32) + 8 * q + 4 * (lane >> 5)
+                                     : wc * WN + grp_c(j, q);
                     u32x2 *p = reinterpret_cast<u32x2 *>(at(dt, r, c));
                     float e[4] = {0.f, 0.f, 0.f, 0.f};
                     uint16_t h[4];
@@ -1083,13 +1323,15 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
 template <int BM, int BN, Stage S, int NW, int D, int KT>
 __global__ __launch_bounds__(64 * NW) void polar_stream_kernel(GemmArgs g) {
     using Geo = StreamGeom<BM, BN, NW, D>;
-    constexpr int kStages = Geo::kStages;
-    __shared__ __attribute__((aligned(1024))) uint16_t smem[kStages * Geo::kStageBytes / 2];
-    // 1 KiB per wave that the ring's idle DMA instructions write (out-of-range
-    // offsets: zeros, no memory traffic) in the last kStages steps of a segment,
-    // so that every step issues the same instructions: no branch around them.
-    __shared__ __attribute__((aligned(1024))) uint16_t sink[NW * 512];
-    __shared__ uint32_t s_arrived;
+    // The ring, then the sink: 1 KiB per wave that the ring's idle DMA instructions write
+    // (out-of-range offsets: zeros, no memory traffic) in the last kStages steps of a
+    // segment, so that every step issues the same instructions: no branch around them.
+    // Last the arrival word; the panel ring fills the LDS and lends its last bytes, which
+    // no epilogue tile covers.
+    constexpr int kWordAt = Geo::kRingBytes + Geo::kSinkBytes - (Geo::kPanelRing ? 16 : 0);
+    __shared__ __attribute__((aligned(1024))) uint16_t smem[(kWordAt + 16) / 2];
+    uint16_t *sink = smem + Geo::kRingBytes / 2;
+    uint32_t &s_arrived = *reinterpret_cast<uint32_t *>(smem + kWordAt / 2);
     const int nk = g.k_steps;
 
     // Work of this workgroup: iterations [it_lo, it_hi) of tiles tile_base + i / nk
@@ -1131,12 +1373,15 @@ __global__ __launch_bounds__(64 * NW) void polar_stream_kernel(GemmArgs g) {
 // halves run the wave-pair kernel (two K chains per output).
 template <Stage S, int KT, int DH>
 __global__ __launch_bounds__(512) void polar_stream_halves_kernel(GemmArgs g) {
-    // ring: two 64 KiB slots for the whole tiles, DH 48 KiB slots for the halves
-    constexpr int kWhole = 2 * StreamGeom<256, 256, 8, 2>::kStageBytes;
-    constexpr int kHalf = DH * StreamGeom<256, 128, 8, DH>::kStageBytes;
-    __shared__ __attribute__((aligned(1024))) uint16_t smem[(kWhole > kHalf ? kWhole : kHalf) / 2];
-    __shared__ __attribute__((aligned(1024))) uint16_t sink[8 * 512];
-    __shared__ uint32_t s_arrived;
+    // ring: five 32 KiB panels for the whole tiles, DH 48 KiB slots for the halves; no
+    // sink in either, and the arrival word is not used
+    using Whole = StreamGeom<256, 256, 8, 2>;
+    using Half = StreamGeom<256, 128, 8, DH>;
+    static_assert(Half::kRingBytes <= Whole::kRingBytes, "the halves' ring fits");
+    static_assert(Whole::kSinkBytes == 0 && Half::kSinkBytes == 0, "no sink");
+    __shared__ __attribute__((aligned(1024))) uint16_t smem[Whole::kRingBytes / 2];
+    uint16_t *sink = smem;
+    uint32_t &s_arrived = *reinterpret_cast<uint32_t *>(smem + Whole::kRingBytes / 2 - 8);
     const int w = static_cast<int>(blockIdx.x);
     const int dp_grid = 8 * g.per_xcd;
     if (w < dp_grid) {

@@ -60,6 +60,16 @@ __device__ __forceinline__ int kc_offset(int row, int chunk) {
     return row * kBK + ((chunk ^ kc_swz(row)) << 3);
 }
 
+// The same for 16x16x32 fragments, whose 16 consecutive rows at one chunk fill the
+// 256-byte bank window: even and odd rows lie in its two halves, so the XOR runs over the
+// row pairs.  It depends on the row modulo 16 alone: the fragments of a wave differ by
+// constant offsets.
+__device__ __forceinline__ int kc_swz16(int row) { return (row >> 1) & 7; }
+
+__device__ __forceinline__ int kc_offset16(int row, int chunk) {
+    return row * kBK + ((chunk ^ kc_swz16(row)) << 3);
+}
+
 // N-contiguous tile [64][BN] (stage-3 X panel, rows = K): chunk c of K-row k is
 // stored at c ^ nc_swz(k).  A transposing read fetches 4 consecutive K-rows by
 // 2 chunks (32 B) per 16-lane group, and a half-wave (two groups: 16 adjacent
@@ -81,6 +91,22 @@ __device__ __forceinline__ int nc_swz(int krow) {
 template <int BN>
 __device__ __forceinline__ int nc_offset(int krow, int chunk) {
     return krow * BN + ((chunk ^ nc_swz<BN>(krow)) << 3);
+}
+
+// The same for 16x16x32 fragments (BN = 128, 192, 256), whose half-wave reads 2 chunks
+// (32 B, at an even chunk) of K-rows k .. k+3 and k+8 .. k+11: bit 3 of k moves the
+// second four rows to the other chunk pair of each 64-byte group, so that the eight
+// rows fill the 256-byte bank window.
+template <int BN>
+__device__ __forceinline__ int nc_swz16(int krow) {
+    static_assert(BN == 128 || BN == 192 || BN == 256, "widths of the 16x16x32 kernels");
+    const int hi = ((krow >> 3) & 1) << 1;
+    if constexpr (BN == 192) return (((krow >> 1) & 1) << 2) | hi;
+    return ((krow & 3) << 2) | hi;
+}
+template <int BN>
+__device__ __forceinline__ int nc_offset16(int krow, int chunk) {
+    return krow * BN + ((chunk ^ nc_swz16<BN>(krow)) << 3);
 }
 
 // ---------------------------------------------------------------------------
@@ -198,6 +224,47 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// v_mfma_f32_16x16x32_bf16: lane l supplies 8 K-values (quarter l/16 of the 32) of row
+// l%16 of A and of column l%16 of B and receives D[4*(l/16) + j][l%16], j = 0..3.  With
+// the K-values in this order its result has the bits of two chained 32x32x16 MFMAs
+// (measured on random inputs over 24 binades), so kernels of either shape agree.
+__device__ __forceinline__ f32x4 mfma_16x16x32(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// LDS byte offsets of the 16x16x32 fragments, as lane parts that a few registers hold and
+// wave-uniform parts that fold into scalars and instruction offsets.
+//
+// K-contiguous tile, k32 slice kk, fragment of rows row0 .. row0+15 (row0 a multiple of
+// 16): (frag16_kc_lane ^ 64 * kk) + 128 * row0.
+__device__ __forceinline__ uint32_t frag16_kc_lane(int lane) {
+    const int r = lane & 15;
+    return static_cast<uint32_t>(r * 128 + (((lane >> 4) ^ kc_swz16(r)) << 4));
+}
+// N-contiguous tile [64][BN], columns n0 .. n0+15 (n0 a multiple of 16): two transposing
+// reads at (frag16_nc_swz ^ 2 * n0) + frag16_nc_row + 64 * BN * kk, and 8 * BN further.
+template <int BN>
+__device__ __forceinline__ uint32_t frag16_nc_swz(int lane) {
+    return static_cast<uint32_t>(nc_swz16<BN>(8 * (lane >> 4) + ((lane & 15) >> 2)) << 4);
+}
+template <int BN>
+__device__ __forceinline__ uint32_t frag16_nc_row(int lane) {
+    const int i = lane & 15;
+    return static_cast<uint32_t>((8 * (lane >> 4) + (i >> 2)) * BN * 2 + 8 * (i & 3));
+}
+using lds_u8 = __attribute__((address_space(3))) uint8_t;
+__device__ __forceinline__ bf16x8 frag16_kc(const lds_u8 *p) {
+    return *reinterpret_cast<const __attribute__((address_space(3))) bf16x8 *>(p);
+}
+template <int BN>
+__device__ __forceinline__ bf16x8 frag16_nc_tr(lds_u8 *p) {
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+        reinterpret_cast<__attribute__((address_space(3))) bf16x4 *>(p));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+        reinterpret_cast<__attribute__((address_space(3))) bf16x4 *>(p + 8 * BN));
+    return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+
 }  // namespace muon_polar
 
 // ===========================================================================
@@ -247,6 +314,18 @@ __device__ __forceinline__ void dma_16B(i32x4 rsrc, uint32_t lds_base, uint32_t 
                  :
                  : "v"(voffset), "s"(rsrc), "{m0}"(__builtin_amdgcn_readfirstlane(lds_base))
                  : "memory");
+}
+
+// The same with the LDS address given as base (wave-uniform) + kOff: the add writes
+// M0 itself, so a group of DMAs into one panel needs one scalar base, not an address
+// each.
+template <uint32_t kOff>
+__device__ __forceinline__ void dma_16B_at(i32x4 rsrc, uint32_t lds_base, uint32_t voffset) {
+    asm volatile("s_add_u32 m0, %1, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %2, 0 offen lds"
+                 :
+                 : "v"(voffset), "s"(__builtin_amdgcn_readfirstlane(lds_base)), "s"(rsrc),
+                   "n"(kOff)
+                 : "memory", "m0", "scc");
 }
 
 // Wait until at most N vector-memory operations of this wave are outstanding,
