@@ -50,7 +50,7 @@ namespace {
 // flight competes with the fragment reads); deeper rings serve latency-bound
 // launches with few K-steps per workgroup, where each step would otherwise wait
 // for one full memory round trip.
-template <int BM, int BN, int NW, int D>
+template <int BM, int BN, int NW, int D, int KT = 0>
 struct StreamGeom {
     static constexpr int kThreads = 64 * NW;
     static constexpr int kABytes = BM * kBK * 2;        // row-operand panel per K-step
@@ -62,15 +62,21 @@ struct StreamGeom {
     static constexpr int kLoads = kLoadsA + kLoadsB;
     static constexpr int kTileBytes = BM * BN * 2;       // bf16 output tile (epilogue)
     static constexpr int kEpiLoads = kTileBytes / 1024 / NW;
+    // Wave pairs: see stream_segment.
+    static constexpr bool kPair = NW == 8 && ((BM == 192 && BN == 192) || (BM == 256 && BN == 128));
+    // Panel ring: 256x256 and 128x128 tiles with 8 waves keep kPanels row and column panels
+    // in turn instead of K-step slots: five (all of the LDS, or half of it for two
+    // workgroups per CU) or, 128x128 with D = 4, nine.  128x128 tiles of two workgroups per
+    // CU keep the slots where rows straddle cache lines (KT: n % 64 != 0), which doubles
+    // the address unit's work: [1,3000,3000] gram 49.8 us with slots, 56.6 with panels.
+    static constexpr bool kPanelRing =
+        NW == 8 && BM == BN && (BM == 256 || (BM == 128 && (D == 4 || KT == 0)));
+    static constexpr int kPanels = D == 2 ? 5 : 9;
     // The epilogue operand tile fits one ring slot (BM, BN <= 128): it is fetched
     // into the first slot the K loop stops refilling, so its latency overlaps the
     // last K-steps instead of following them.
-    static constexpr bool kEpiInSlot = kTileBytes <= kStageBytes && D >= 3;
-    // Wave pairs (see stream_segment) and the 256x256 tiles with 8 waves, whose ring holds
-    // five 32 KiB panels (all of the LDS) instead of K-step slots.
-    static constexpr bool kPair = NW == 8 && ((BM == 192 && BN == 192) || (BM == 256 && BN == 128));
-    static constexpr bool kPanelRing = BM == 256 && BN == 256 && NW == 8;
-    static constexpr int kRingBytes = kPanelRing ? 5 * kABytes : D * kStageBytes;
+    static constexpr bool kEpiInSlot = kTileBytes <= kStageBytes && D >= 3 && !kPanelRing;
+    static constexpr int kRingBytes = kPanelRing ? kPanels * kABytes : D * kStageBytes;
     // 1 KiB per wave past the ring that idle DMA instructions write, where a ring slot may
     // hold the epilogue tile meanwhile (kEpiInSlot) or for the kernels they share code with.
     static constexpr int kSinkBytes = kPair || kPanelRing ? 0 : NW * 1024;
@@ -137,7 +143,7 @@ template <int BM, int BN, Stage S, int NW, int D, int KT, bool DG = false>
 __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem, uint16_t *sink,
                                                uint32_t *s_arrived_p, int unit, int tile_base,
                                                int lt, int kbeg, int kend, int half = -1) {
-    using Geo = StreamGeom<BM, BN, NW, D>;
+    using Geo = StreamGeom<BM, BN, NW, D, KT>;
     constexpr int kThreads = Geo::kThreads;
     // Wave pairs (8 waves on a 192x192 tile, whose 2 x 4 wave grid would not be
     // made of 32-wide MFMA blocks, or on a 256x128 apply tile, whose 2 x 4 grid
@@ -164,7 +170,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
                   "diagonal pairs: 64x64 tiles of a triangular stage, 4 waves");
     constexpr int WM = BM / 2, WN = DG ? BN : BN / (kGridWaves / 2);
     constexpr bool kPanelRing = Geo::kPanelRing;
-    constexpr int kPanels = 5;
+    constexpr int kPanels = Geo::kPanels;
     // MFMA shape: 16x16x32 in the large-tile kernels (256x256 with 8 waves, the wave
     // pairs), else 32x32x16.  The large tiles run at the power limit (the clock falls as
     // the MFMA pipe fills), and 16x16x32 takes less power per FLOP: a loop of MFMAs alone
@@ -686,65 +692,76 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     if constexpr (kPanelRing) {
         // Per K-step k (panels A_k, B_k), k32 slices s0 and s1:
         //   mfma(s0) + frags(s1) | wait panels k+1, barrier | mfma(s1) + frags(next s0)
-        // The barrier frees A_k's and B_k's places: column panel B_{k+2} then row panel
-        // A_{k+3} stream into them, one DMA instruction every kGap MFMAs over slice s1 and
-        // the next step's s0.  Issued together behind the barrier, the 64 instructions of
-        // a step (16 clocks each in the CU's address unit, half of a step's MFMA time)
-        // queue up and hold the waves' MFMAs back: MFMA pipe busy 68% of apply's cycles at
-        // [4096,14336] with two 64 KiB slots, 78% spread.  The half step more than two
-        // slots hold gives the spread panels time to land (8 MFMAs apart: 351 us; 4: 359).
+        // The barrier frees A_k's and B_k's places, and the panels due there stream in one
+        // DMA instruction every kGap MFMAs over slice s1 and the next step's s0.  Issued
+        // together behind the barrier, a step's instructions (256x256: 64 of 16 clocks
+        // each in the CU's address unit, half of the step's MFMA time) queue up and hold
+        // the waves' MFMAs back: MFMA pipe busy 68% of apply's cycles at [4096,14336] with
+        // two 64 KiB slots, 78% spread.  The half step that five panels hold beyond two
+        // slots gives them time to land (8 MFMAs apart: 351 us; 4: 359).  128x128 tiles,
+        // five panels against two slots: [8,512,2048] apply 14.7 -> 13.3 us, [1,2560,4096]
+        // apply 68.6 -> 58.6, [32,1024,1024] step 173.7 -> 157.5; nine against four slots:
+        // [1,1024,4096] apply 14.4 -> 11.5, [1,2560,4096] gram 34.1 -> 29.0.
         // Idle instructions past the segment's end write zeros to places nothing reads.
         static_assert(Geo::kABytes == Geo::kBBytes, "panel ring");
         constexpr int kL = Geo::kLoadsA, kP = Geo::kABytes, kM = kMfmaPerSlice;
         constexpr int kGap = kM / kL;
-        static_assert((2 * kL - 1) * kGap < 2 * kM, "a group is issued before the next barrier");
+        static_assert((2 * kL - 1) * kGap < 2 * kM && kM <= kL * kGap,
+                      "a group is issued before the next barrier, its second panel past slice s1");
         const uint32_t wave_dst = smem_base + wave * kL * 1024;
         auto wrap = [](int p) { return p >= kPanels ? p - kPanels : p; };
-        // DMA instruction due after MFMA q of a group: column panel of step sb into position
-        // pos_b, then row panel of step sb + 1 into position pos_a.
-        auto group_at = [&](auto qc, int sb, int pos_b, int pos_a) {
+        // Panels alternate A_0, B_0, A_1, ...; panel p lives at position p mod kPanels (odd).
+        // Step k frees the places of A_k and B_k, where panels kPanels further land: column
+        // panel B_{k+kAhead}, then row panel A_{k+kAhead+1}.
+        static_assert(kPanels % 2 == 1, "a step's freed places take a column then a row panel");
+        constexpr int kAhead = kPanels / 2;
+        auto dma_panel = [&](auto jc, auto row_c, int step, int pos) {
+            constexpr int j = decltype(jc)::value;
+            if constexpr (decltype(row_c)::value)
+                dma_16B_at<j * 1024>(rs_row, wave_dst + pos * kP, a_voff(j, step, step < kend));
+            else
+                dma_16B_at<j * 1024>(rs_col, wave_dst + pos * kP, b_voff(j, step, step < kend));
+        };
+        // DMA instruction due after MFMA q of a step's group.
+        auto group_at = [&](auto qc, int step_b, int pos_b, int pos_a) {
             constexpr int q = decltype(qc)::value, j = q / kGap;
             if constexpr (q % kGap == 0 && j < kL)
-                dma_16B_at<j * 1024>(rs_col, wave_dst + pos_b * kP, b_voff(j, sb, sb < kend));
+                dma_panel(std::integral_constant<int, j>{}, std::false_type{}, step_b, pos_b);
             else if constexpr (q % kGap == 0 && j < 2 * kL)
-                dma_16B_at<(j - kL) * 1024>(rs_row, wave_dst + pos_a * kP,
-                                            a_voff(j - kL, sb + 1, sb + 1 < kend));
+                dma_panel(std::integral_constant<int, j - kL>{}, std::true_type{}, step_b + 1,
+                          pos_a);
         };
-        static_for<kL>([&](auto jc) {
-            constexpr int j = decltype(jc)::value;
-            dma_16B_at<j * 1024>(rs_row, wave_dst, a_voff(j, kbeg, true));
+        static_for<kPanels - 2>([&](auto pc) {
+            constexpr int pn = decltype(pc)::value;
+            static_for<kL>([&](auto jc) {
+                dma_panel(jc, std::integral_constant<bool, pn % 2 == 0>{}, kbeg + pn / 2, pn);
+            });
         });
-        static_for<kL>([&](auto jc) {
-            constexpr int j = decltype(jc)::value;
-            dma_16B_at<j * 1024>(rs_col, wave_dst + kP, b_voff(j, kbeg, true));
-        });
-        static_for<kL>([&](auto jc) {
-            constexpr int j = decltype(jc)::value;
-            dma_16B_at<j * 1024>(rs_row, wave_dst + 2 * kP, a_voff(j, kbeg + 1, 1 < nkl));
-        });
-        static_for<kM>([&](auto mc) { group_at(mc, kbeg + 1, 3, 4); });
+        static_for<kM>([&](auto mc) { group_at(mc, kbeg + kAhead - 1, kPanels - 2, kPanels - 1); });
         if (tail_fix && nkl == 1) {  // the segment is the tile's last K-step alone
             wait_vm<0>();
             fix_tail(0, kP);
         }
-        wait_vm_barrier<kL + (kM + kGap - 1) / kGap>();
+        wait_vm_barrier<(kPanels - 3) * kL>();
         bf16x8 fr0[SM], fc0[SN], fr1[SM], fc1[SN];
         load_frags(0, kP, 0, fr0, fc0);
         int pa = 0, k = 0;
         auto step = [&](auto ax_c) {
-            const int pb = wrap(pa + 1), na = wrap(pa + 2), nb = wrap(pa + 3), pz = wrap(pa + 4);
+            const int pb = wrap(pa + 1), na = wrap(pa + 2), nb = wrap(pa + 3);
+            // the places step k - 1 freed
+            const int fb = wrap(pa + kPanels - 2), fa = wrap(pa + kPanels - 1);
             if constexpr (decltype(ax_c)::value) add_ax(pa * kP, pb * kP, kbeg + k);
             mfma_slice(fr0, fc0, pa * kP, pb * kP, 1, fr1, fc1, [&](auto mc) {
-                group_at(std::integral_constant<int, kM + decltype(mc)::value>{}, kbeg + k + 1,
-                         nb, pz);
+                group_at(std::integral_constant<int, kM + decltype(mc)::value>{},
+                         kbeg + k - 1 + kAhead, fb, fa);
             });
             if (tail_fix && k == nkl - 2) {
                 wait_vm<0>();
                 fix_tail(na * kP, nb * kP);
             }
-            wait_vm_barrier<kL>();
+            wait_vm_barrier<(kPanels - 4) * kL>();
             mfma_slice(fr1, fc1, na * kP, nb * kP, 0, fr0, fc0,
-                       [&](auto mc) { group_at(mc, kbeg + k + 2, pa, pb); });
+                       [&](auto mc) { group_at(mc, kbeg + k + kAhead, pa, pb); });
             pa = na;
             ++k;
         };
@@ -1322,7 +1339,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
 
 template <int BM, int BN, Stage S, int NW, int D, int KT>
 __global__ __launch_bounds__(64 * NW) void polar_stream_kernel(GemmArgs g) {
-    using Geo = StreamGeom<BM, BN, NW, D>;
+    using Geo = StreamGeom<BM, BN, NW, D, KT>;
     // The ring, then the sink: 1 KiB per wave that the ring's idle DMA instructions write
     // (out-of-range offsets: zeros, no memory traffic) in the last kStages steps of a
     // segment, so that every step issues the same instructions: no branch around them.
@@ -1375,8 +1392,8 @@ template <Stage S, int KT, int DH>
 __global__ __launch_bounds__(512) void polar_stream_halves_kernel(GemmArgs g) {
     // ring: five 32 KiB panels for the whole tiles, DH 48 KiB slots for the halves; no
     // sink in either, and the arrival word is not used
-    using Whole = StreamGeom<256, 256, 8, 2>;
-    using Half = StreamGeom<256, 128, 8, DH>;
+    using Whole = StreamGeom<256, 256, 8, 2, KT>;
+    using Half = StreamGeom<256, 128, 8, DH, KT>;
     static_assert(Half::kRingBytes <= Whole::kRingBytes, "the halves' ring fits");
     static_assert(Whole::kSinkBytes == 0 && Half::kSinkBytes == 0, "no sink");
     __shared__ __attribute__((aligned(1024))) uint16_t smem[Whole::kRingBytes / 2];

@@ -1,7 +1,7 @@
-"""The K loops of the large-tile kernels at their shortest lengths: 256x256 tiles (the ring
-of five panels) and 192x192 wave pairs (two and three slots) over 1 to 6 K-steps, every
-K mask and both forms.  256x256 tiles accumulate in the 64x64 kernels' order: the same
-bits.  Wave pairs sum two K chains: exact-sum inputs, bitwise against the 64x64 kernels."""
+"""The K loops of the large-tile kernels at their shortest lengths: 256x256 and 128x128
+tiles (rings of five and nine panels) and 192x192 wave pairs (two and three slots) over 1
+to 6 K-steps, every K mask and both forms.  The panel rings accumulate in the 64x64
+kernels' order: the same bits.  Wave pairs sum two K chains: exact-sum inputs, bitwise against the 64x64 kernels."""
 
 from __future__ import annotations
 
@@ -38,13 +38,15 @@ SMALL = {"MUON_POLAR_GRAM_TILE": "64", "MUON_POLAR_POLY_TILE": "64", "MUON_POLAR
          "MUON_POLAR_DIAG_PAIRS": "0"}
 
 
+@pytest.mark.parametrize("tile,depth", [("256", "2"), ("128", "2"), ("128", "4")])
 @pytest.mark.parametrize("shape", SHAPES)
-def test_256_tiles_equal_64_tiles(monkeypatch, shape):
+def test_panel_rings_equal_64_tiles(monkeypatch, shape, tile, depth):
     import muon_ascend950  # noqa: F401
 
     x = O.make_input(shape, seed=51).to(DEV)
-    big = {"MUON_POLAR_GRAM_TILE": "256", "MUON_POLAR_POLY_TILE": "256",
-           "MUON_POLAR_APPLY_TILE_M": "256"}
+    big = {f"MUON_POLAR_{s}_DEPTH": depth for s in ("GRAM", "POLY", "APPLY")}
+    big.update({"MUON_POLAR_GRAM_TILE": tile, "MUON_POLAR_POLY_TILE": tile,
+                "MUON_POLAR_APPLY_TILE_M": tile})
     assert torch.equal(_step(monkeypatch, x, C0, big), _step(monkeypatch, x, C0, SMALL))
 
 
