@@ -11,6 +11,7 @@
 #include "muon_polar.h"
 
 #include <hip/hip_runtime_api.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <climits>
@@ -52,6 +53,22 @@ uint64_t env_u64(const char *name, uint64_t def, bool *present = nullptr) {
     return end != v ? static_cast<uint64_t>(parsed) : def;
 }
 
+// Whether a MUON_POLAR_* variable that tunes the stage kernels is set (any but those that
+// leave them as they are).
+bool stage_knob_set() {
+    static const char *const kOthers[] = {"DEBUG_SYNC=", "CAPI_LIBRARY=", "RESIDENT="};
+    constexpr char kPrefix[] = "MUON_POLAR_";
+    constexpr size_t kLen = sizeof(kPrefix) - 1;
+    for (char **e = environ; e != nullptr && *e != nullptr; ++e) {
+        if (std::strncmp(*e, kPrefix, kLen) != 0) continue;
+        bool other = false;
+        for (const char *name : kOthers)
+            other = other || std::strncmp(*e + kLen, name, std::strlen(name)) == 0;
+        if (!other) return true;
+    }
+    return false;
+}
+
 int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 size_t align256(size_t v) { return (v + 255u) & ~size_t(255u); }
 
@@ -74,6 +91,8 @@ struct Knobs {
     uint32_t sk_pieces;     // most stream-K pieces per cut tile (0: by tile size, sk_max_pieces)
     uint32_t y_cpol, ap_cpol;  // cache policy of the DMA-fed kernels' Y / A and P stores
                                // (GemmArgs::out_cpol)
+    uint32_t resident;  // 1: small matrices run whole steps in one workgroup each
+                        // (polar_resident.hip); off when a stage knob is set
     bool operator==(const Knobs &o) const {
         return gram_tile == o.gram_tile && poly_tile == o.poly_tile && apply_bm == o.apply_bm &&
                apply_bn == o.apply_bn && stream == o.stream && stream_k == o.stream_k &&
@@ -81,7 +100,7 @@ struct Knobs {
                depth[2] == o.depth[2] && pair == o.pair && halves == o.halves &&
                halves_depth == o.halves_depth && diag_pairs == o.diag_pairs &&
                sk_rounds == o.sk_rounds && sk_share == o.sk_share && sk_pieces == o.sk_pieces && y_cpol == o.y_cpol &&
-               ap_cpol == o.ap_cpol;
+               ap_cpol == o.ap_cpol && resident == o.resident;
     }
 };
 
@@ -117,6 +136,7 @@ struct PlanKeyHash {
         mix(k.knobs.halves_depth);
         mix(k.knobs.diag_pairs);
         mix(k.knobs.sk_rounds);
+        mix(k.knobs.resident);
         mix(uint64_t(k.knobs.sk_pieces) << 32 | uint64_t(k.knobs.sk_share) << 16 | uint64_t(k.knobs.y_cpol) << 8 | k.knobs.ap_cpol);
         return static_cast<size_t>(h);
     }
@@ -143,6 +163,7 @@ struct Plan {
     int64_t gram_grid, poly_grid, apply_grid;
     size_t gram_bytes, workspace_bytes;
     bool stream;
+    bool resident;  // steps run in polar_resident.hip's kernel (the stage calls never do)
     int y_cpol, ap_cpol;  // store cache policies (GemmArgs::out_cpol)
     int waves[3];  // waves per workgroup of the DMA-fed kernel of each stage
     int depth[3];  // LDS ring slots of the DMA-fed kernel of each stage
@@ -260,6 +281,9 @@ int read_knobs(int64_t batch, int64_t m, int64_t n, int cus, Knobs &k) {
     k.waves = static_cast<uint32_t>(env_u64("MUON_POLAR_WAVES", kDefaultWaves));
     if (k.waves != 4 && k.waves != 8)
         return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_WAVES must be 4 or 8");
+    k.resident = static_cast<uint32_t>(env_u64("MUON_POLAR_RESIDENT", 1));
+    if (k.resident > 1) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_RESIDENT must be 0 or 1");
+    if (stage_knob_set()) k.resident = 0;
     k.pair = static_cast<uint32_t>(env_u64("MUON_POLAR_PAIR", 1));
     if (k.pair > 1) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_PAIR must be 0 or 1");
     k.halves = static_cast<uint32_t>(env_u64("MUON_POLAR_APPLY_HALVES", 1));
@@ -467,6 +491,31 @@ struct Target {
 // the offset 2^31, which is only out of range for buffers below that size.
 constexpr int64_t kMaxMatrixElems = int64_t(1) << 30;
 
+// Whether the steps of [batch, m, n] run in the resident kernel (polar_resident.hip).  Its
+// time grows with the matrix, on one CU; that of the stage kernels' three launches is
+// nearly constant for a small batch.  Both in units of 10 ns, as measured: a step takes
+// base + slope per 32 columns by the shorter side's 32-row blocks; launch, load and store
+// 360, or 350 and 10 per 1000 elements where vectors are scattered in LDS (a tall matrix,
+// rows of n % 8 != 0 elements).  The stage kernels take 1440 for rows of whole vectors,
+// 1380 tall, 1640 for even and 1780 for odd rows (the padded copy).  Steps, resident
+// against stages: [64,64] 5.4 / 12.5 us, [129,130] 12.2 / 15.8, [3,129,257] 17.2 / 18.1,
+// [128,384] 13.6 / 14.3, left to the stages [128,480] 15.4 / 15.1, [150,271] 18.3 / 17.6,
+// tall [384,128] 17.4 / 14.0.  From 64 matrices on the stages' tiles add up ([64,192,192]
+// 17.0 / 19.1, [300,160,256] 31 / 66, [600,96,400] 39 / 92).  A single step decides, not a
+// chain (which gains more): both take one route, so a chain's results are its steps'.
+bool resident_pays(int64_t batch, int64_t m, int64_t n) {
+    if (muon_polar::resident_fit(m, n) == 0) return false;
+    if (batch >= 256) return true;
+    static constexpr int kBase[muon_polar::kResidentBlocks + 1] = {0, 150, 170, 320, 300, 410, 520};
+    static constexpr int kSlope[muon_polar::kResidentBlocks + 1] = {0, 14, 26, 33, 54, 75, 110};
+    const int64_t nb = ceil_div(std::min(m, n), 32), lb = ceil_div(std::max(m, n), 32);
+    const bool scattered = m > n || n % 8 != 0;
+    const int64_t cost =
+        kBase[nb] + kSlope[nb] * lb + (scattered ? 350 + m * n / 100 : 360);
+    const int64_t stages = m > n ? 1380 : n % 8 == 0 ? 1440 : n % 2 == 0 ? 1640 : 1780;
+    return cost <= (batch >= 64 ? 2000 : stages);
+}
+
 int build_plan(int64_t batch, int64_t m, int64_t n, const Knobs &knobs, const Target &tgt,
                Plan &out) {
     const bool tall = m > n;
@@ -497,6 +546,7 @@ int build_plan(int64_t batch, int64_t m, int64_t n, const Knobs &knobs, const Ta
     // The right-Gram stages exist only as DMA-fed kernels: MUON_POLAR_STREAM=0
     // selects the register-staged kernels for m <= n alone.
     p.stream = knobs.stream != 0 || tall;
+    p.resident = knobs.resident != 0 && resident_pays(batch, m, n);
     p.y_cpol = static_cast<int>(knobs.y_cpol);
     p.ap_cpol = static_cast<int>(knobs.ap_cpol);
     if (p.gram_grid >= (int64_t(1) << 31) || p.apply_grid >= (int64_t(1) << 31))
@@ -1090,6 +1140,30 @@ int pad_input(const Plan &p, void *workspace, const void *x, int64_t batch, hipS
     return MUON_POLAR_OK;
 }
 
+// Whether the plan runs `steps` steps (after the normalisation, if asked) in one launch
+// of the resident kernel.
+bool resident_runs(const Plan &p, int64_t batch, int64_t steps, bool normalize) {
+    return p.resident && steps >= 1 && steps <= muon_polar::kResidentSteps &&
+           (!normalize || muon_polar::norm_chunk(batch, p.m * p.n) == 4096);
+}
+
+// vec: the normalisation's 16-byte order (launch_normalize).
+int run_resident(const Plan &p, const void *x, void *y, int64_t batch, const double *coefficients,
+                 int64_t steps, bool normalize, bool vec, hipStream_t stream) {
+    muon_polar::ResidentArgs g{};
+    g.x = static_cast<const uint16_t *>(x);
+    g.y = static_cast<uint16_t *>(y);
+    g.m = static_cast<int32_t>(p.m);
+    g.n = static_cast<int32_t>(p.n);
+    g.tall = p.tall ? 1 : 0;
+    g.steps = static_cast<int32_t>(steps);
+    g.normalize = normalize ? 1 : 0;
+    g.vec = vec ? 1 : 0;
+    g.chunks = normalize ? static_cast<int32_t>(muon_polar::norm_chunks(batch, p.m * p.n)) : 0;
+    for (int64_t i = 0; i < 3 * steps; ++i) g.coef[i] = static_cast<float>(coefficients[i]);
+    return finish_stage(muon_polar::launch_resident(g, batch, stream), stream, "resident");
+}
+
 // One step given the workspace: left form (m <= n) or right-Gram form; rows the
 // DMA-fed kernels cannot read in place are first copied into the zero-padded
 // buffer (pad_input).
@@ -1099,6 +1173,10 @@ int pad_input(const Plan &p, void *workspace, const void *x, int64_t batch, hipS
 int run_step(const Plan &p, const void *x, void *y, void *workspace, int64_t batch, double a,
              double b, double c, hipStream_t stream, int64_t ldx_in = 0, int64_t n_out = 0,
              bool force_pad = false) {
+    if (p.resident && ldx_in == 0 && n_out == 0) {
+        const double coef[3] = {a, b, c};
+        return run_resident(p, x, y, batch, coef, 1, false, false, stream);
+    }
     char *ws = static_cast<char *>(workspace);
     void *gram = ws;
     void *poly = ws + align256(p.gram_bytes);
@@ -1571,9 +1649,11 @@ int muon_polar_express(const void *x, void *y, void *workspace, size_t workspace
     auto iterate = [&](int64_t i) { return (steps - i) % 2 == 0 ? out : scratch; };
 
     const uint16_t *cur = static_cast<const uint16_t *>(x);
+    const bool vec = (m * n) % 8 == 0 && aligned16(x) && aligned16(iterate(0));
+    if (resident_runs(p, batch, steps, normalize != 0))
+        return run_resident(p, x, y, batch, coefficients, steps, normalize != 0, vec, stream);
     if (normalize) {
         uint16_t *dst = iterate(0);
-        const bool vec = (m * n) % 8 == 0 && aligned16(x) && aligned16(dst);
         st = finish_stage(muon_polar::launch_normalize(cur, dst, partial, batch, m * n, vec, stream),
                           stream, "normalize");
         if (st != MUON_POLAR_OK) return st;
@@ -1629,8 +1709,10 @@ int muon_polar_muon_update(void *param, const void *grad, void *momentum_buffer,
     // The normalised input goes where the iterate chain starts (out for an even
     // step count, else scratch); the momentum pass writes the other buffer, which
     // the first step overwrites only after the normalisation has read it.
+    // (The resident kernel normalises by itself, from the scratch buffer.)
+    const bool resident = resident_runs(p, batch, steps, true);
     uint16_t *first = steps % 2 == 0 ? out : scratch;
-    uint16_t *x0 = steps % 2 == 0 ? scratch : out;
+    uint16_t *x0 = steps % 2 == 0 || resident ? scratch : out;
     const int64_t mn = m * n;
     const bool vec = mn % 8 == 0 && aligned16(grad) && aligned16(momentum_buffer);
     st = finish_stage(
@@ -1640,11 +1722,15 @@ int muon_polar_muon_update(void *param, const void *grad, void *momentum_buffer,
                                          static_cast<float>(momentum), nesterov != 0, vec, stream),
         stream, "momentum");
     if (st != MUON_POLAR_OK) return st;
-    st = finish_stage(muon_polar::launch_norm_scale(x0, first, partial, batch, mn, mn % 8 == 0,
-                                                    stream),
-                      stream, "normalize");
-    if (st != MUON_POLAR_OK) return st;
-    st = run_steps(p, workspace, first, out, scratch, batch, coefficients, steps, stream);
+    if (resident) {
+        st = run_resident(p, x0, out, batch, coefficients, steps, true, mn % 8 == 0, stream);
+    } else {
+        st = finish_stage(muon_polar::launch_norm_scale(x0, first, partial, batch, mn, mn % 8 == 0,
+                                                        stream),
+                          stream, "normalize");
+        if (st != MUON_POLAR_OK) return st;
+        st = run_steps(p, workspace, first, out, scratch, batch, coefficients, steps, stream);
+    }
     if (st != MUON_POLAR_OK) return st;
     const int64_t total = batch * mn;
     return finish_stage(

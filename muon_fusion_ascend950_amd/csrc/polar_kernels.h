@@ -151,6 +151,22 @@ hipError_t launch_pad_rows(const uint16_t *x, uint16_t *xp, int64_t rows, int64_
 hipError_t launch_muon_param_update(float *p, const uint16_t *o, int64_t total, float decay,
                                     float alpha, bool vec, hipStream_t stream);
 
+// Whole steps of small matrices, one workgroup each (polar_resident.hip).  x and y are
+// [batch, m, n] dense, any alignment; steps coefficient triples in coef; normalize: the
+// per-matrix normalisation first, in chunks of 4096 elements (norm_chunk must be 4096;
+// vec as launch_normalize's).
+constexpr int kResidentSteps = 8;
+constexpr int kResidentBlocks = 6;  // 32-row blocks of the shorter side
+struct ResidentArgs {
+    const uint16_t *x;
+    uint16_t *y;
+    int32_t m, n, tall, steps, normalize, vec, chunks;
+    float coef[3 * kResidentSteps];
+};
+// KiB of LDS the kernel for [m, n] matrices uses (80 or 160), 0 when they do not fit.
+int resident_fit(int64_t m, int64_t n);
+hipError_t launch_resident(const ResidentArgs &g, int64_t batch, hipStream_t stream);
+
 // Scratch of the allocation-free step (polar_noalloc.hip): a device array of
 // kNoAllocScratchBytes per GPU.  noalloc_scratch returns its address on
 // `device`, which must be the current device (looked up once per device).

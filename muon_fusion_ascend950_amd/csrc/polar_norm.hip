@@ -21,6 +21,7 @@
 // number of 64-element K-steps: X [rows, n] -> Xp [rows, np], np a multiple of 8
 // (of 64 as used), the columns n .. np-1 zero, one 16-byte chunk of Xp per thread.
 #include "polar_kernels.h"
+#include "polar_norm.hpp"
 #include "polar_tile.hpp"
 
 namespace muon_polar {
@@ -38,15 +39,10 @@ constexpr int kNormUnroll = 4;      // norm passes: 16 bytes per thread and iter
 constexpr int kMomentumUnroll = 2;  // momentum pass: 64 bytes per thread and iteration
 constexpr int kParamUnroll = 2;     // parameter pass: 48 bytes per thread and iteration
 
-__device__ __forceinline__ float bf16_round(float v) {
-    return bf16_bits_to_f32(f32_to_bf16_bits(v));
-}
-
 // Sum of v over the block in a fixed order: butterfly within each wave, then the
 // four wave totals in index order.  `red` holds 4 floats of LDS.
 __device__ __forceinline__ float block_sum(float v, float *red) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    v = wave_sum(v);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (lane == 0) red[wave] = v;
     __syncthreads();
@@ -77,12 +73,7 @@ __global__ __launch_bounds__(kNormThreads) void norm_partial_kernel(const uint16
             for (int u = 0; u < kNormUnroll; ++u) {
                 if (e + u * kNormStride >= e1) break;
 #pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const float lo = bf16_bits_to_f32(v[u][w] & 0xffffu);
-                    const float hi = bf16_bits_to_f32(v[u][w] >> 16);
-                    acc = fmaf(lo, lo, acc);
-                    acc = fmaf(hi, hi, acc);
-                }
+                for (int w = 0; w < 4; ++w) acc = add_squares(acc, v[u][w]);
             }
         }
     } else {
@@ -105,9 +96,7 @@ __global__ __launch_bounds__(kNormThreads) void norm_scale_kernel(const uint16_t
     const int b = blockIdx.x / chunks, c = blockIdx.x - b * chunks;
     float s = 0.0f;
     for (int i = threadIdx.x; i < chunks; i += kNormThreads) s += partial[int64_t(b) * chunks + i];
-    const float total = block_sum(s, red);
-    const float norm = bf16_round(sqrtf(total));
-    const float d = bf16_round(bf16_round(norm * 1.01f) + 1e-6f);
+    const float d = norm_divisor(block_sum(s, red));
 
     const uint16_t *xb = x + int64_t(b) * mn;
     uint16_t *yb = y + int64_t(b) * mn;
