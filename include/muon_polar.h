@@ -202,6 +202,21 @@ int muon_polar_muon_update(void *param, const void *grad, void *momentum_buffer,
                            int64_t steps, double lr, double weight_decay, double lr_scale,
                            hipStream_t stream);
 
+/* The same update of `count` tensors that lie apart, in one batch: params[i], grads[i]
+ * and momentum_buffers[i] are [matrices, m, n], row-major contiguous, fp32 (grads bf16
+ * with grad_bf16 != 0).  Results are those of muon_polar_muon_update on the batch of
+ * count·matrices matrices.  The pointer arrays are read during the call only.  Every
+ * param and buffer and the workspace are disjoint from each other and from every grad;
+ * grads may share memory.  `workspace` must hold the info.muon_workspace_bytes of batch
+ * count·matrices.
+ * No reference counterpart (as muon_polar_muon_update). */
+int muon_polar_muon_update_list(void *const *params, const void *const *grads, int grad_bf16,
+                                void *const *momentum_buffers, int64_t count, void *workspace,
+                                size_t workspace_bytes, int64_t matrices, int64_t m, int64_t n,
+                                double momentum, int nesterov, const double *coefficients,
+                                int64_t steps, double lr, double weight_decay, double lr_scale,
+                                hipStream_t stream);
+
 /* Host-side check of a launch plan (test support; no reference counterpart).
  * Builds the plan muon_polar_step would use for [batch, m, n] on a device of
  * `cus` compute units with blocks_per_cu[s] resident workgroups per CU for the

@@ -64,10 +64,15 @@ def load_library() -> None:
                          weight_decay, lr_scale):
         return None
 
+    def fake_muon_update_list(params, grads, momentum_buffers, momentum, nesterov, coefficients,
+                              lr, weight_decay, lr_scale):
+        return None
+
     for name, fake in (("muon_ascend950::polar_step", fake_polar_step),
                        ("muon_ascend950::polar_step_tall", fake_polar_step),
                        ("muon_ascend950::polar_express", fake_polar_express),
-                       ("muon_ascend950::muon_update", fake_muon_update)):
+                       ("muon_ascend950::muon_update", fake_muon_update),
+                       ("muon_ascend950::muon_update_list", fake_muon_update_list)):
         try:
             torch.library.register_fake(name)(fake)
         except RuntimeError as exc:

@@ -21,6 +21,7 @@ EXPORTED_FUNCTIONS = (
     "muon_polar_apply",
     "muon_polar_express",
     "muon_polar_muon_update",
+    "muon_polar_muon_update_list",
     "muon_polar_check_plan",
     "muon_polar_last_error",
     "muon_polar_version",
@@ -99,12 +100,17 @@ def load() -> ctypes.CDLL:
     lib.muon_polar_muon_update.argtypes = [vp, vp, vp, vp, sz, i64, i64, i64, dbl, ctypes.c_int,
                                            ctypes.POINTER(ctypes.c_double), i64, dbl, dbl, dbl,
                                            vp]
+    ptrs = ctypes.POINTER(ctypes.c_void_p)
+    lib.muon_polar_muon_update_list.argtypes = [ptrs, ptrs, ctypes.c_int, ptrs, i64, vp, sz, i64,
+                                                i64, i64, dbl, ctypes.c_int,
+                                                ctypes.POINTER(ctypes.c_double), i64, dbl, dbl,
+                                                dbl, vp]
     lib.muon_polar_check_plan.argtypes = [i64, i64, i64, ctypes.c_int,
                                           ctypes.POINTER(ctypes.c_int), ctypes.POINTER(PlanExtents)]
     for name in ("muon_polar_query", "muon_polar_step", "muon_polar_step_noalloc",
                  "muon_polar_gram", "muon_polar_poly",
                  "muon_polar_apply", "muon_polar_express", "muon_polar_muon_update",
-                 "muon_polar_check_plan"):
+                 "muon_polar_muon_update_list", "muon_polar_check_plan"):
         getattr(lib, name).restype = ctypes.c_int
     lib.muon_polar_last_error.argtypes = []
     lib.muon_polar_last_error.restype = ctypes.c_char_p

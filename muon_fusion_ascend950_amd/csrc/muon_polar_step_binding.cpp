@@ -160,6 +160,55 @@ void MuonUpdateHip(const at::Tensor &param, const at::Tensor &grad,
     TORCH_CHECK(st == MUON_POLAR_OK, "muon_update: ", muon_polar_last_error());
 }
 
+// The same update of parameters of one shape [..., M, N] in tensors of their own, as one
+// batch; gradients fp32 or bf16.
+void MuonUpdateListHip(at::TensorList params, at::TensorList grads, at::TensorList buffers,
+                       double momentum, bool nesterov, at::ArrayRef<double> coefficients,
+                       double lr, double weight_decay, double lr_scale) {
+    TORCH_CHECK(!params.empty() && grads.size() == params.size() && buffers.size() == params.size(),
+                "muon_update_list: params, grads and momentum_buffers must be lists of one length");
+    const at::Tensor &first = params[0];
+    TORCH_CHECK(first.device().is_cuda(), "muon_update_list: tensors must be ROCm (HIP) device tensors");
+    TORCH_CHECK(first.dim() >= 2 && first.numel() > 0,
+                "muon_update_list: tensors must be non-empty matrices");
+    const at::ScalarType grad_type = grads[0].scalar_type();
+    TORCH_CHECK(grad_type == at::kFloat || grad_type == at::kBFloat16,
+                "muon_update_list: grads must be float32 or bfloat16");
+    std::vector<void *> p, b;
+    std::vector<const void *> g;
+    for (size_t i = 0; i < params.size(); ++i) {
+        for (const at::Tensor *t : {&params[i], &grads[i], &buffers[i]}) {
+            TORCH_CHECK(t->device() == first.device(), "muon_update_list: tensors must share one device");
+            TORCH_CHECK(t->sizes() == first.sizes(), "muon_update_list: tensors must have one shape");
+            TORCH_CHECK(t->is_contiguous(), "muon_update_list: tensors must be contiguous");
+        }
+        TORCH_CHECK(params[i].scalar_type() == at::kFloat && buffers[i].scalar_type() == at::kFloat,
+                    "muon_update_list: params and momentum_buffers must be float32");
+        TORCH_CHECK(grads[i].scalar_type() == grad_type, "muon_update_list: grads must have one dtype");
+        p.push_back(params[i].data_ptr());
+        g.push_back(grads[i].data_ptr());
+        b.push_back(buffers[i].data_ptr());
+    }
+    TORCH_CHECK(coefficients.size() % 3 == 0,
+                "muon_update_list: coefficients must be (a, b, c) triples");
+    const c10::OptionalDeviceGuard device_guard(first.device());
+    const int64_t m = first.size(-2), n = first.size(-1), matrices = first.numel() / (m * n);
+    const int64_t count = static_cast<int64_t>(p.size());
+    muon_polar_shape_info info{};
+    int st = muon_polar_query(count * matrices, m, n, &info);
+    TORCH_CHECK(st == MUON_POLAR_OK, "muon_update_list: ", muon_polar_last_error());
+    at::Tensor workspace = at::empty({static_cast<int64_t>(info.muon_workspace_bytes)},
+                                     first.options().dtype(at::kByte));
+    hipStream_t stream = c10::hip::getCurrentHIPStream(first.device().index()).stream();
+    st = muon_polar_muon_update_list(p.data(), g.data(), grad_type == at::kBFloat16 ? 1 : 0,
+                                     b.data(), count, workspace.data_ptr(),
+                                     info.muon_workspace_bytes, matrices, m, n, momentum,
+                                     nesterov ? 1 : 0, coefficients.data(),
+                                     static_cast<int64_t>(coefficients.size() / 3), lr,
+                                     weight_decay, lr_scale, stream);
+    TORCH_CHECK(st == MUON_POLAR_OK, "muon_update_list: ", muon_polar_last_error());
+}
+
 }  // namespace
 
 TORCH_LIBRARY(muon_ascend950, m) {
@@ -168,6 +217,9 @@ TORCH_LIBRARY(muon_ascend950, m) {
     m.def("polar_express(Tensor x, float[] coefficients, bool normalize) -> Tensor");
     m.def("muon_update(Tensor(a!) param, Tensor grad, Tensor(b!) momentum_buffer, float momentum, "
           "bool nesterov, float[] coefficients, float lr, float weight_decay, float lr_scale) -> ()");
+    m.def("muon_update_list(Tensor(a!)[] params, Tensor[] grads, Tensor(b!)[] momentum_buffers, "
+          "float momentum, bool nesterov, float[] coefficients, float lr, float weight_decay, "
+          "float lr_scale) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(muon_ascend950, CUDA, m) {
@@ -175,4 +227,5 @@ TORCH_LIBRARY_IMPL(muon_ascend950, CUDA, m) {
     m.impl("polar_step_tall", &MuonPolarStepTallHip);
     m.impl("polar_express", &MuonPolarExpressHip);
     m.impl("muon_update", &MuonUpdateHip);
+    m.impl("muon_update_list", &MuonUpdateListHip);
 }

@@ -1235,6 +1235,104 @@ int run_steps(const Plan &p, void *workspace, const uint16_t *cur, uint16_t *out
     return MUON_POLAR_OK;
 }
 
+// The Muon update of muon_polar_muon_update and muon_polar_muon_update_list.
+int update_tensors(const muon_polar::MuonTensors &t, void *workspace, size_t workspace_bytes,
+                   int64_t m, int64_t n, double momentum, int nesterov,
+                   const double *coefficients, int64_t steps, double lr, double weight_decay,
+                   double lr_scale, hipStream_t stream) {
+    for (int64_t i = 0; i < t.count; ++i)
+        if (t.param[i] == nullptr || t.grad[i] == nullptr || t.buf[i] == nullptr)
+            return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "null pointer");
+    if (steps < 0) return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "steps must be >= 0");
+    if (steps > 0 && coefficients == nullptr)
+        return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "coefficients is null");
+    if (!std::isfinite(momentum) || momentum < 0.0 || momentum > 1.0)
+        return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "momentum must be in [0, 1]");
+    if (!std::isfinite(lr) || !std::isfinite(weight_decay) || !std::isfinite(lr_scale))
+        return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "lr, weight_decay and lr_scale must be finite");
+    const int64_t batch = t.count * t.matrices;
+    Plan p{};
+    int st = get_plan(batch, m, n, p);
+    if (st != MUON_POLAR_OK) return st;
+    if (workspace == nullptr || workspace_bytes < p.muon_workspace_bytes)
+        return fail(MUON_POLAR_ERR_WORKSPACE,
+                    "workspace must hold " + std::to_string(p.muon_workspace_bytes) +
+                        " bytes, got " + std::to_string(workspace == nullptr ? 0 : workspace_bytes));
+    if (!aligned16(workspace))
+        return fail(MUON_POLAR_ERR_WORKSPACE, "workspace must be 16-byte aligned");
+    // What is written (every param and buf, the workspace) is disjoint from all else;
+    // gradients may share memory with one another.
+    struct Range {
+        uintptr_t lo, hi;
+        bool written;
+    };
+    const uintptr_t f32_bytes = static_cast<uintptr_t>(t.matrices * m * n * 4);
+    const uintptr_t g_bytes = t.grad_bf16 ? f32_bytes / 2 : f32_bytes;
+    std::vector<Range> ranges;
+    ranges.reserve(static_cast<size_t>(3 * t.count + 1));
+    auto add = [&](const void *q, uintptr_t bytes, bool written) {
+        const uintptr_t lo = reinterpret_cast<uintptr_t>(q);
+        ranges.push_back({lo, lo + bytes, written});
+    };
+    add(workspace, static_cast<uintptr_t>(p.muon_workspace_bytes), true);
+    bool vec_gb = true, vec_p = true;
+    for (int64_t i = 0; i < t.count; ++i) {
+        add(t.param[i], f32_bytes, true);
+        add(t.grad[i], g_bytes, false);
+        add(t.buf[i], f32_bytes, true);
+        vec_gb = vec_gb && aligned16(t.grad[i]) && aligned16(t.buf[i]);
+        vec_p = vec_p && aligned16(t.param[i]);
+    }
+    std::sort(ranges.begin(), ranges.end(),
+              [](const Range &x, const Range &y) { return x.lo < y.lo; });
+    uintptr_t end_any = 0, end_written = 0;
+    for (const Range &r : ranges) {
+        if (r.lo < (r.written ? end_any : end_written))
+            return fail(MUON_POLAR_ERR_INVALID_ARGUMENT,
+                        "param, grad, momentum_buffer and workspace must not overlap");
+        end_any = std::max(end_any, r.hi);
+        if (r.written) end_written = std::max(end_written, r.hi);
+    }
+
+    char *ws = static_cast<char *>(workspace);
+    uint16_t *out = reinterpret_cast<uint16_t *>(ws + p.muon_o_offset);
+    uint16_t *scratch = reinterpret_cast<uint16_t *>(ws + p.express_x_offset);
+    if (p.tall && steps > 0) {
+        st = check_tall(p, out, scratch);
+        if (st != MUON_POLAR_OK) return st;
+    }
+    float *partial = reinterpret_cast<float *>(ws + p.express_norm_offset);
+    // The normalised input goes where the iterate chain starts (out for an even
+    // step count, else scratch); the momentum pass writes the other buffer, which
+    // the first step overwrites only after the normalisation has read it.
+    // (The resident kernel normalises by itself, from the scratch buffer.)
+    const bool resident = resident_runs(p, batch, steps, true);
+    uint16_t *first = steps % 2 == 0 ? out : scratch;
+    uint16_t *x0 = steps % 2 == 0 || resident ? scratch : out;
+    const int64_t mn = m * n;
+    st = finish_stage(
+        muon_polar::launch_muon_momentum(t, x0, partial, mn, static_cast<float>(1.0 - momentum),
+                                         static_cast<float>(momentum), nesterov != 0,
+                                         mn % 8 == 0 && vec_gb, stream),
+        stream, "momentum");
+    if (st != MUON_POLAR_OK) return st;
+    if (resident) {
+        st = run_resident(p, x0, out, batch, coefficients, steps, true, mn % 8 == 0, stream);
+    } else {
+        st = finish_stage(muon_polar::launch_norm_scale(x0, first, partial, batch, mn, mn % 8 == 0,
+                                                        stream),
+                          stream, "normalize");
+        if (st != MUON_POLAR_OK) return st;
+        st = run_steps(p, workspace, first, out, scratch, batch, coefficients, steps, stream);
+    }
+    if (st != MUON_POLAR_OK) return st;
+    return finish_stage(
+        muon_polar::launch_muon_param_update(t, out, mn, static_cast<float>(1.0 - lr * weight_decay),
+                                             static_cast<float>(-lr * lr_scale),
+                                             t.matrices * mn % 8 == 0 && vec_p, stream),
+        stream, "param update");
+}
+
 int reject_tall_stage(int64_t m, int64_t n) {
     if (m > n)
         return fail(MUON_POLAR_ERR_INVALID_ARGUMENT,
@@ -1667,77 +1765,26 @@ int muon_polar_muon_update(void *param, const void *grad, void *momentum_buffer,
                            int64_t n, double momentum, int nesterov, const double *coefficients,
                            int64_t steps, double lr, double weight_decay, double lr_scale,
                            hipStream_t stream) {
-    if (param == nullptr || grad == nullptr || momentum_buffer == nullptr)
-        return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "null pointer");
-    if (steps < 0) return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "steps must be >= 0");
-    if (steps > 0 && coefficients == nullptr)
-        return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "coefficients is null");
-    if (!std::isfinite(momentum) || momentum < 0.0 || momentum > 1.0)
-        return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "momentum must be in [0, 1]");
-    if (!std::isfinite(lr) || !std::isfinite(weight_decay) || !std::isfinite(lr_scale))
-        return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "lr, weight_decay and lr_scale must be finite");
-    Plan p{};
-    int st = get_plan(batch, m, n, p);
-    if (st != MUON_POLAR_OK) return st;
-    if (workspace == nullptr || workspace_bytes < p.muon_workspace_bytes)
-        return fail(MUON_POLAR_ERR_WORKSPACE,
-                    "workspace must hold " + std::to_string(p.muon_workspace_bytes) +
-                        " bytes, got " + std::to_string(workspace == nullptr ? 0 : workspace_bytes));
-    if (!aligned16(workspace))
-        return fail(MUON_POLAR_ERR_WORKSPACE, "workspace must be 16-byte aligned");
-    // fp32 param, grad and buffer, and the workspace: pairwise disjoint
-    const uintptr_t f32_bytes = static_cast<uintptr_t>(batch * m * n * 4);
-    const uintptr_t lo[4] = {reinterpret_cast<uintptr_t>(param), reinterpret_cast<uintptr_t>(grad),
-                             reinterpret_cast<uintptr_t>(momentum_buffer),
-                             reinterpret_cast<uintptr_t>(workspace)};
-    const uintptr_t len[4] = {f32_bytes, f32_bytes, f32_bytes,
-                              static_cast<uintptr_t>(p.muon_workspace_bytes)};
-    for (int i = 0; i < 4; ++i)
-        for (int j = i + 1; j < 4; ++j)
-            if (lo[i] < lo[j] + len[j] && lo[j] < lo[i] + len[i])
-                return fail(MUON_POLAR_ERR_INVALID_ARGUMENT,
-                            "param, grad, momentum_buffer and workspace must not overlap");
+    const muon_polar::MuonTensors t{&param, &grad, &momentum_buffer, 1, batch, false};
+    return update_tensors(t, workspace, workspace_bytes, m, n, momentum, nesterov, coefficients,
+                          steps, lr, weight_decay, lr_scale, stream);
+}
 
-    char *ws = static_cast<char *>(workspace);
-    uint16_t *out = reinterpret_cast<uint16_t *>(ws + p.muon_o_offset);
-    uint16_t *scratch = reinterpret_cast<uint16_t *>(ws + p.express_x_offset);
-    if (p.tall && steps > 0) {
-        st = check_tall(p, out, scratch);
-        if (st != MUON_POLAR_OK) return st;
-    }
-    float *partial = reinterpret_cast<float *>(ws + p.express_norm_offset);
-    // The normalised input goes where the iterate chain starts (out for an even
-    // step count, else scratch); the momentum pass writes the other buffer, which
-    // the first step overwrites only after the normalisation has read it.
-    // (The resident kernel normalises by itself, from the scratch buffer.)
-    const bool resident = resident_runs(p, batch, steps, true);
-    uint16_t *first = steps % 2 == 0 ? out : scratch;
-    uint16_t *x0 = steps % 2 == 0 || resident ? scratch : out;
-    const int64_t mn = m * n;
-    const bool vec = mn % 8 == 0 && aligned16(grad) && aligned16(momentum_buffer);
-    st = finish_stage(
-        muon_polar::launch_muon_momentum(static_cast<const float *>(grad),
-                                         static_cast<float *>(momentum_buffer), x0, partial, batch,
-                                         mn, static_cast<float>(1.0 - momentum),
-                                         static_cast<float>(momentum), nesterov != 0, vec, stream),
-        stream, "momentum");
-    if (st != MUON_POLAR_OK) return st;
-    if (resident) {
-        st = run_resident(p, x0, out, batch, coefficients, steps, true, mn % 8 == 0, stream);
-    } else {
-        st = finish_stage(muon_polar::launch_norm_scale(x0, first, partial, batch, mn, mn % 8 == 0,
-                                                        stream),
-                          stream, "normalize");
-        if (st != MUON_POLAR_OK) return st;
-        st = run_steps(p, workspace, first, out, scratch, batch, coefficients, steps, stream);
-    }
-    if (st != MUON_POLAR_OK) return st;
-    const int64_t total = batch * mn;
-    return finish_stage(
-        muon_polar::launch_muon_param_update(
-            static_cast<float *>(param), out, total, static_cast<float>(1.0 - lr * weight_decay),
-            static_cast<float>(-lr * lr_scale), total % 8 == 0 && aligned16(param), stream),
-        stream, "param update");
+int muon_polar_muon_update_list(void *const *params, const void *const *grads, int grad_bf16,
+                                void *const *momentum_buffers, int64_t count, void *workspace,
+                                size_t workspace_bytes, int64_t matrices, int64_t m, int64_t n,
+                                double momentum, int nesterov, const double *coefficients,
+                                int64_t steps, double lr, double weight_decay, double lr_scale,
+                                hipStream_t stream) {
+    if (params == nullptr || grads == nullptr || momentum_buffers == nullptr)
+        return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "null pointer");
+    if (count <= 0 || matrices <= 0 || count > (int64_t(1) << 31) / matrices)
+        return fail(MUON_POLAR_ERR_INVALID_ARGUMENT,
+                    "count and matrices must be positive and their product below 2^31");
+    const muon_polar::MuonTensors t{params,   grads,    momentum_buffers,
+                                    count,    matrices, grad_bf16 != 0};
+    return update_tensors(t, workspace, workspace_bytes, m, n, momentum, nesterov, coefficients,
+                          steps, lr, weight_decay, lr_scale, stream);
 }
 
 int muon_polar_check_plan(int64_t batch, int64_t m, int64_t n, int cus, const int *blocks_per_cu,

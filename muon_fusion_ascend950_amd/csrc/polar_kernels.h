@@ -135,21 +135,36 @@ hipError_t launch_normalize(const uint16_t *x, uint16_t *y, float *partial, int6
 hipError_t launch_norm_scale(const uint16_t *x, uint16_t *y, const float *partial,
                              int64_t batch, int64_t mn, bool vec, hipStream_t stream);
 
+// The tensors of one Muon update: `count` of each, of `matrices` m × n matrices; tensor
+// i's matrices are i·matrices .. of the batch.  param and buf fp32, grad fp32 or bf16.
+struct MuonTensors {
+    void *const *param;
+    const void *const *grad;
+    void *const *buf;
+    int64_t count;
+    int64_t matrices;
+    bool grad_bf16;
+};
+
+// Matrices (momentum pass) or tensors (parameter pass) of one launch whose pointers
+// travel in its arguments: 2 KiB of the 4 KiB that a launch takes.
+constexpr int kMuonListMax = 128;
+
 // Muon update passes (polar_norm.hip).  Momentum: buf ← lerp(buf, g, w),
 // g' = nesterov ? lerp(g, buf, beta) : buf, x0 = bf16(g'), and x0's per-chunk
 // sums of squares into `partial` in launch_normalize's order (ready for
-// launch_norm_scale).  vec: mn % 8 == 0 and 16-byte aligned g, buf, x0.
-hipError_t launch_muon_momentum(const float *g, float *buf, uint16_t *x0, float *partial,
-                                int64_t batch, int64_t mn, float w, float beta, bool nesterov,
-                                bool vec, hipStream_t stream);
+// launch_norm_scale).  vec: mn % 8 == 0 and every g and buf 16-byte aligned (x0 is).
+hipError_t launch_muon_momentum(const MuonTensors &t, uint16_t *x0, float *partial, int64_t mn,
+                                float w, float beta, bool nesterov, bool vec, hipStream_t stream);
 // Xp [rows, np] = X [rows, n] with zero columns n .. np-1 (np >= n, np % 8 == 0,
 // 16-byte aligned xp).
 hipError_t launch_pad_rows(const uint16_t *x, uint16_t *xp, int64_t rows, int64_t n, int64_t np,
                            hipStream_t stream);
 
-// p ← p·decay + alpha·O over `total` elements; vec: total % 8 == 0, 16-byte aligned.
-hipError_t launch_muon_param_update(float *p, const uint16_t *o, int64_t total, float decay,
-                                    float alpha, bool vec, hipStream_t stream);
+// p ← p·decay + alpha·O over every tensor; vec: a whole number of 8 elements in each,
+// 16-byte aligned.
+hipError_t launch_muon_param_update(const MuonTensors &t, const uint16_t *o, int64_t mn,
+                                    float decay, float alpha, bool vec, hipStream_t stream);
 
 // Whole steps of small matrices, one workgroup each (polar_resident.hip).  x and y are
 // [batch, m, n] dense, any alignment; steps coefficient triples in coef; normalize: the

@@ -136,22 +136,90 @@ __device__ __forceinline__ float lerp_rounded(float start, float end, float w) {
     return fabsf(w) < 0.5f ? start + w * (end - start) : end - (end - start) * (1.0f - w);
 }
 
+// Where matrix b of the Muon update's fp32 tensors (and of its gradient, G = float or
+// the bits of a bf16) lies: rows of one batched tensor, or tensors of their own, whose
+// pointers travel in the kernel arguments (no table in memory to fill and to wait for).
+template <typename G>
+struct BatchedMats {
+    const G *g;
+    float *w;
+    int64_t mn;
+    __device__ __forceinline__ const G *grad(int b) const { return g + int64_t(b) * mn; }
+    __device__ __forceinline__ float *buf(int b) const { return w + int64_t(b) * mn; }
+};
+template <typename G>
+struct ListedMats {
+    const G *g[kMuonListMax];
+    float *w[kMuonListMax];
+    __device__ __forceinline__ const G *grad(int b) const { return g[b]; }
+    __device__ __forceinline__ float *buf(int b) const { return w[b]; }
+};
+struct BatchedParam {
+    float *p;
+    __device__ __forceinline__ float *at(int) const { return p; }
+};
+struct ListedParams {
+    float *p[kMuonListMax];
+    __device__ __forceinline__ float *at(int b) const { return p[b]; }
+};
+
+// 8 consecutive gradient values as fp32 (exact for bf16); kVec: 16-byte aligned.
+template <bool kVec>
+__device__ __forceinline__ void load8(const float *g, float (&v)[8]) {
+    if (kVec) {
+        const f32x4 lo = *reinterpret_cast<const f32x4 *>(g);
+        const f32x4 hi = *reinterpret_cast<const f32x4 *>(g + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = lo[i];
+            v[i + 4] = hi[i];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = g[i];
+    }
+}
+template <bool kVec>
+__device__ __forceinline__ void load8(const uint16_t *g, float (&v)[8]) {
+    if (kVec) {
+        const u32x4 w = *reinterpret_cast<const u32x4 *>(g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[2 * i] = bf16_bits_to_f32(w[i] & 0xffffu);
+            v[2 * i + 1] = bf16_bits_to_f32(w[i] >> 16);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = bf16_bits_to_f32(g[i]);
+    }
+}
+__device__ __forceinline__ float grad_value(float g) { return g; }
+__device__ __forceinline__ float grad_value(uint16_t g) { return bf16_bits_to_f32(g); }
+
 // Momentum pass of the Muon update over chunk c of matrix b (chunks as in
 // norm_partial_kernel):
 //     buf ← lerp(buf, g, w)                  (w = 1 − momentum)
 //     g'  = lerp(g, buf, momentum) | buf     (Nesterov or plain)
 //     x0  = bf16(g'),   partial[b, c] = Σ x0²  in norm_partial_kernel's order
-// order8: mn % 8 == 0 (8 consecutive elements per thread and step, the vector
-// path's order); vec: also 16-byte aligned g, buf and x0 (vector accesses).
-template <bool kOrder8, bool kVec>
+// kOrder8: mn % 8 == 0 (8 consecutive elements per thread and step, the vector
+// path's order); kVec: also 16-byte aligned g, buf and x0 (vector accesses).
+//
+// Bound by HBM: 12 bytes per element of an fp32 gradient, 10 of a bf16 one, and the
+// 2 of x0.  Separate tensors are read and written where they lie: gathering them into
+// one batch and copying the results back moved 40 bytes per element more (with the
+// parameter pass's) in two launches per tensor: an optimizer step over [768,768] x 8,
+// [3072,768] x 2 and [768,3072] x 2 took 841 us with it and takes 655; the update of one
+// [1024,4096] with a bf16 gradient 218 us with an fp32 copy of it, 206 without.
+template <bool kOrder8, bool kVec, typename G, typename Mats>
 __global__ __launch_bounds__(kNormThreads) void muon_momentum_kernel(
-    const float *__restrict__ g, float *__restrict__ buf, uint16_t *__restrict__ x0,
-    float *__restrict__ partial, int64_t mn, int chunks, int64_t chunk, float w, float beta,
-    int nesterov) {
+    const Mats mats, uint16_t *__restrict__ x0, float *__restrict__ partial, int64_t mn,
+    int chunks, int64_t chunk, float w, float beta, int nesterov) {
 #pragma clang fp contract(off)
     __shared__ float red[4];
     const int b = blockIdx.x / chunks, c = blockIdx.x - b * chunks;
     const int64_t base = int64_t(b) * mn;
+    const G *__restrict__ gb = mats.grad(b);
+    float *__restrict__ bufb = mats.buf(b);
     const int64_t e0 = int64_t(c) * chunk;
     const int64_t e1 = e0 + chunk < mn ? e0 + chunk : mn;
     float acc = 0.0f;
@@ -172,23 +240,8 @@ __global__ __launch_bounds__(kNormThreads) void muon_momentum_kernel(
             for (int u = 0; u < kU; ++u) {
                 const int64_t eu = e + u * kNormStride;
                 if (eu >= e1) break;
-                if (kVec) {
-                    const f32x4 g0 = *reinterpret_cast<const f32x4 *>(g + base + eu);
-                    const f32x4 g1 = *reinterpret_cast<const f32x4 *>(g + base + eu + 4);
-                    const f32x4 b0 = *reinterpret_cast<const f32x4 *>(buf + base + eu);
-                    const f32x4 b1 = *reinterpret_cast<const f32x4 *>(buf + base + eu + 4);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        gv[u][i] = g0[i]; gv[u][i + 4] = g1[i];
-                        bv[u][i] = b0[i]; bv[u][i + 4] = b1[i];
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        gv[u][i] = g[base + eu + i];
-                        bv[u][i] = buf[base + eu + i];
-                    }
-                }
+                load8<kVec>(gb + eu, gv[u]);
+                load8<kVec>(static_cast<const float *>(bufb + eu), bv[u]);
             }
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
@@ -199,8 +252,8 @@ __global__ __launch_bounds__(kNormThreads) void muon_momentum_kernel(
 #pragma unroll
                 for (int i = 0; i < 8; ++i) nb[i] = one(gv[u][i], bv[u][i], h[i]);
                 if (kVec) {
-                    *reinterpret_cast<f32x4 *>(buf + base + eu) = f32x4{nb[0], nb[1], nb[2], nb[3]};
-                    *reinterpret_cast<f32x4 *>(buf + base + eu + 4) =
+                    *reinterpret_cast<f32x4 *>(bufb + eu) = f32x4{nb[0], nb[1], nb[2], nb[3]};
+                    *reinterpret_cast<f32x4 *>(bufb + eu + 4) =
                         f32x4{nb[4], nb[5], nb[6], nb[7]};
                     store16_sc1(rs_x0, static_cast<uint32_t>((eu - e0) * 2),
                                 u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16),
@@ -208,7 +261,7 @@ __global__ __launch_bounds__(kNormThreads) void muon_momentum_kernel(
                 } else {
 #pragma unroll
                     for (int i = 0; i < 8; ++i) {
-                        buf[base + eu + i] = nb[i];
+                        bufb[eu + i] = nb[i];
                         x0[base + eu + i] = static_cast<uint16_t>(h[i]);
                     }
                 }
@@ -217,7 +270,7 @@ __global__ __launch_bounds__(kNormThreads) void muon_momentum_kernel(
     } else {
         for (int64_t e = e0 + threadIdx.x; e < e1; e += kNormThreads) {
             uint32_t h;
-            buf[base + e] = one(g[base + e], buf[base + e], h);
+            bufb[e] = one(grad_value(gb[e]), bufb[e], h);
             x0[base + e] = static_cast<uint16_t>(h);
         }
     }
@@ -225,13 +278,15 @@ __global__ __launch_bounds__(kNormThreads) void muon_momentum_kernel(
     if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// p ← p·decay + alpha·O over `total` elements (fp32 p, bf16 O; each product and
-// the sum rounded on their own).
-template <bool kVec>
+// p ← p·decay + alpha·O over `total` elements of tensor blockIdx.y (fp32 p, bf16 O;
+// each product and the sum rounded on their own).
+template <bool kVec, typename Params>
 __global__ __launch_bounds__(kNormThreads) void muon_param_update_kernel(
-    float *__restrict__ p, const uint16_t *__restrict__ o, int64_t total, float decay,
+    const Params params, const uint16_t *__restrict__ o_all, int64_t total, float decay,
     float alpha) {
 #pragma clang fp contract(off)
+    float *__restrict__ p = params.at(blockIdx.y);
+    const uint16_t *__restrict__ o = o_all + int64_t(blockIdx.y) * total;
     const int64_t stride = int64_t(gridDim.x) * kNormThreads * 8;
     if (kVec) {
         // kParamUnroll grid strides per trip, every load of the trip issued first
@@ -351,34 +406,94 @@ hipError_t launch_norm_scale(const uint16_t *x, uint16_t *y, const float *partia
                            dim3(static_cast<unsigned>(grid)), dim3(kNormThreads), a2, 0, stream);
 }
 
-hipError_t launch_muon_momentum(const float *g, float *buf, uint16_t *x0, float *partial,
-                                int64_t batch, int64_t mn, float w, float beta, bool nesterov,
+namespace {
+
+template <typename G, typename Mats>
+hipError_t launch_momentum_pass(const Mats &mats, uint16_t *x0, float *partial, int64_t matrices,
+                                int64_t mn, int64_t chunk, float w, float beta, bool nesterov,
                                 bool vec, hipStream_t stream) {
-    int64_t chunk = norm_chunk(batch, mn);
-    const int64_t chunks = norm_chunks(batch, mn);
-    const int64_t grid = batch * chunks;
+    const int64_t chunks = (mn + chunk - 1) / chunk;
+    const int64_t grid = matrices * chunks;
     if (grid <= 0 || grid >= (int64_t(1) << 31)) return hipErrorInvalidValue;
+    const void *fn =
+        mn % 8 != 0 ? reinterpret_cast<const void *>(&muon_momentum_kernel<false, false, G, Mats>)
+        : vec       ? reinterpret_cast<const void *>(&muon_momentum_kernel<true, true, G, Mats>)
+                    : reinterpret_cast<const void *>(&muon_momentum_kernel<true, false, G, Mats>);
     int ch = static_cast<int>(chunks), nv = nesterov ? 1 : 0;
-    void *args[] = {&g, &buf, &x0, &partial, &mn, &ch, &chunk, &w, &beta, &nv};
-    const bool order8 = mn % 8 == 0;
-    const void *fn = order8 ? (vec ? reinterpret_cast<const void *>(&muon_momentum_kernel<true, true>)
-                                   : reinterpret_cast<const void *>(&muon_momentum_kernel<true, false>))
-                            : reinterpret_cast<const void *>(&muon_momentum_kernel<false, false>);
+    void *args[] = {const_cast<Mats *>(&mats), &x0, &partial, &mn, &ch, &chunk, &w, &beta, &nv};
     return hipLaunchKernel(fn, dim3(static_cast<unsigned>(grid)), dim3(kNormThreads), args, 0,
                            stream);
 }
 
-hipError_t launch_muon_param_update(float *p, const uint16_t *o, int64_t total, float decay,
-                                    float alpha, bool vec, hipStream_t stream) {
-    if (total <= 0) return hipErrorInvalidValue;
+template <typename G>
+hipError_t momentum_of(const MuonTensors &t, uint16_t *x0, float *partial, int64_t mn, float w,
+                       float beta, bool nesterov, bool vec, hipStream_t stream) {
+    const int64_t matrices = t.count * t.matrices;
+    const int64_t chunk = norm_chunk(matrices, mn);
+    if (t.count == 1) {
+        const BatchedMats<G> mats{static_cast<const G *>(t.grad[0]), static_cast<float *>(t.buf[0]),
+                                  mn};
+        return launch_momentum_pass<G>(mats, x0, partial, matrices, mn, chunk, w, beta, nesterov,
+                                       vec, stream);
+    }
+    for (int64_t i0 = 0; i0 < matrices; i0 += kMuonListMax) {
+        const int64_t cnt = matrices - i0 < kMuonListMax ? matrices - i0 : kMuonListMax;
+        ListedMats<G> mats{};
+        for (int64_t i = 0; i < cnt; ++i) {
+            const int64_t k = (i0 + i) / t.matrices, off = ((i0 + i) % t.matrices) * mn;
+            mats.g[i] = static_cast<const G *>(t.grad[k]) + off;
+            mats.w[i] = static_cast<float *>(t.buf[k]) + off;
+        }
+        hipError_t e = launch_momentum_pass<G>(mats, x0 + i0 * mn,
+                                               partial + i0 * ((mn + chunk - 1) / chunk), cnt, mn,
+                                               chunk, w, beta, nesterov, vec, stream);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+template <typename Params>
+hipError_t launch_param_pass(const Params &params, const uint16_t *o, int64_t tensors,
+                             int64_t total, float decay, float alpha, bool vec,
+                             hipStream_t stream) {
     // 8 elements per thread; at most 8 waves' worth of blocks per CU on 256 CUs,
     // a grid-stride loop beyond that
     const int64_t blocks = (total + kNormThreads * 8 - 1) / (kNormThreads * 8);
-    const unsigned grid = static_cast<unsigned>(blocks < 4096 ? blocks : 4096);
-    void *args[] = {&p, &o, &total, &decay, &alpha};
-    const void *fn = vec ? reinterpret_cast<const void *>(&muon_param_update_kernel<true>)
-                         : reinterpret_cast<const void *>(&muon_param_update_kernel<false>);
-    return hipLaunchKernel(fn, dim3(grid), dim3(kNormThreads), args, 0, stream);
+    const int64_t most = (4096 + tensors - 1) / tensors;
+    void *args[] = {const_cast<Params *>(&params), &o, &total, &decay, &alpha};
+    const void *fn = vec ? reinterpret_cast<const void *>(&muon_param_update_kernel<true, Params>)
+                         : reinterpret_cast<const void *>(&muon_param_update_kernel<false, Params>);
+    return hipLaunchKernel(
+        fn, dim3(static_cast<unsigned>(blocks < most ? blocks : most), static_cast<unsigned>(tensors)),
+        dim3(kNormThreads), args, 0, stream);
+}
+
+}  // namespace
+
+hipError_t launch_muon_momentum(const MuonTensors &t, uint16_t *x0, float *partial, int64_t mn,
+                                float w, float beta, bool nesterov, bool vec,
+                                hipStream_t stream) {
+    return t.grad_bf16
+               ? momentum_of<uint16_t>(t, x0, partial, mn, w, beta, nesterov, vec, stream)
+               : momentum_of<float>(t, x0, partial, mn, w, beta, nesterov, vec, stream);
+}
+
+hipError_t launch_muon_param_update(const MuonTensors &t, const uint16_t *o, int64_t mn,
+                                    float decay, float alpha, bool vec, hipStream_t stream) {
+    const int64_t per_tensor = t.matrices * mn;
+    if (t.count <= 0 || per_tensor <= 0) return hipErrorInvalidValue;
+    if (t.count == 1)
+        return launch_param_pass(BatchedParam{static_cast<float *>(t.param[0])}, o, 1, per_tensor,
+                                 decay, alpha, vec, stream);
+    for (int64_t i0 = 0; i0 < t.count; i0 += kMuonListMax) {
+        const int64_t cnt = t.count - i0 < kMuonListMax ? t.count - i0 : kMuonListMax;
+        ListedParams params{};
+        for (int64_t i = 0; i < cnt; ++i) params.p[i] = static_cast<float *>(t.param[i0 + i]);
+        hipError_t e = launch_param_pass(params, o + i0 * per_tensor, cnt, per_tensor, decay, alpha,
+                                         vec, stream);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_normalize(const uint16_t *x, uint16_t *y, float *partial, int64_t batch,

@@ -26,7 +26,8 @@ from .ops import COEFFICIENTS
 # Muon.step batches parameters of one shape into one native call when each matrix is
 # small (at most _GROUP_MAX_NUMEL elements): a small matrix alone leaves most CUs idle
 # and its steps are latency-bound, while a batch of them runs in about the time of one.
-# Batches hold at most _GROUP_BATCH_NUMEL elements (bounding the stacked copies).
+# Batches hold at most _GROUP_BATCH_NUMEL elements (bounding the workspace and, where
+# the tensors cannot be updated where they lie, the stacked copies).
 _GROUP_MAX_NUMEL = 1 << 22
 _GROUP_BATCH_NUMEL = 1 << 24
 
@@ -46,6 +47,46 @@ def _flat(coefficients, steps: int):
     return flat
 
 
+class _Matrices:
+    """Tensors of one shape that lie apart, in the place of their stack."""
+
+    def __init__(self, tensors):
+        self.tensors = list(tensors)
+        self.shape = torch.Size((len(self.tensors), *self.tensors[0].shape))
+
+
+def _updatable_in_place(params, grads, bufs) -> bool:
+    """Whether the native update can read and write these tensors where they lie:
+    ordinary contiguous GPU tensors of one shape, gradients of one dtype, and nothing
+    that is written shares memory with another tensor.  A tall matrix whose width is no
+    multiple of 8 has no native form (its update runs on the transposed matrix), and
+    traced programs keep to the operations on tensors."""
+    shape, device, dtype = params[0].shape, params[0].device, grads[0].dtype
+    if (torch.compiler.is_compiling() or device.type != "cuda" or len(shape) < 2
+            or 0 in shape or dtype not in (torch.float32, torch.bfloat16)
+            or (shape[-2] > shape[-1] and shape[-1] % 8 != 0)):
+        return False
+    ranges = []
+    for tensors, want, written in ((params, torch.float32, True), (grads, dtype, False),
+                                   (bufs, torch.float32, True)):
+        for t in tensors:
+            if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != want
+                    or t.shape != shape or t.device != device or not t.is_contiguous()
+                    or t.is_neg()):
+                return False
+            start = t.data_ptr()
+            ranges.append((start, start + t.numel() * t.element_size(), written))
+    ranges.sort()
+    end_any = end_written = 0
+    for start, end, written in ranges:
+        if start < (end_any if written else end_written):
+            return False
+        end_any = max(end_any, end)
+        if written:
+            end_written = max(end_written, end)
+    return True
+
+
 @torch.no_grad()
 def muon_update(param: torch.Tensor, grad: torch.Tensor, momentum_buffer: torch.Tensor, *,
                 lr: float, momentum: float = 0.95, nesterov: bool = True,
@@ -57,6 +98,13 @@ def muon_update(param: torch.Tensor, grad: torch.Tensor, momentum_buffer: torch.
     a batch of matrices); grad: same shape, float32 or bfloat16.  ``lr_scale``
     defaults to ``sqrt(max(1, M / N))``.
     """
+    if isinstance(param, _Matrices):
+        rows, cols = param.shape[-2:]
+        scale = default_lr_scale(rows, cols) if lr_scale is None else float(lr_scale)
+        torch.ops.muon_ascend950.muon_update_list(
+            param.tensors, grad.tensors, momentum_buffer.tensors, float(momentum), bool(nesterov),
+            _flat(coefficients, ns_steps), float(lr), float(weight_decay), scale)
+        return
     for name, t in (("param", param), ("grad", grad), ("momentum_buffer", momentum_buffer)):
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"{name} must be a torch.Tensor")
@@ -75,6 +123,13 @@ def muon_update(param: torch.Tensor, grad: torch.Tensor, momentum_buffer: torch.
     rows, cols = param.shape[-2], param.shape[-1]
     scale = default_lr_scale(rows, cols) if lr_scale is None else float(lr_scale)
     flat = _flat(coefficients, ns_steps)
+
+    # a bfloat16 gradient is read as it is, with no float32 copy
+    if grad.dtype == torch.bfloat16 and _updatable_in_place([param], [grad], [momentum_buffer]):
+        torch.ops.muon_ascend950.muon_update_list([param], [grad], [momentum_buffer],
+                                                  float(momentum), bool(nesterov), flat, float(lr),
+                                                  float(weight_decay), scale)
+        return
 
     def as3d(t):
         return t.reshape(-1, rows, cols)
@@ -110,8 +165,8 @@ class Muon(torch.optim.Optimizer):
     the momentum buffer is float32, created at the first step.
 
     ``group_shapes``: parameters of one group that share a shape and a device, each of
-    at most 4M elements, are stacked and updated in one batched call (as nanochat's
-    Muon stacks same-shape parameters), in batches of at most 16M elements; each is
+    at most 4M elements, are updated in one batched call (nanochat's Muon stacks
+    same-shape parameters), in batches of at most 16M elements; each is
     updated exactly as alone except that the batch's launch plan may cut the
     iteration's sums differently (fp32 rounding of O; the momentum buffers are the
     same bits).
@@ -166,15 +221,24 @@ class Muon(torch.optim.Optimizer):
         return loss
 
     def _update_stacked(self, ps, kw) -> None:
-        """One batched update of same-shape parameters: stacked copies of the
-        parameters, gradients and buffers go through one native call and are copied
-        back (a single parameter is updated in place)."""
+        """One batched update of same-shape parameters, where they lie if the native call
+        can take them so; otherwise stacked copies of the parameters, gradients and
+        buffers go through it and are copied back (a single parameter is updated in
+        place)."""
         bufs = [self.state[p]["momentum_buffer"] for p in ps]
         if len(ps) == 1:
             muon_update(ps[0], ps[0].grad, bufs[0], **kw)
             return
+        grads = [p.grad for p in ps]
+        if _updatable_in_place(ps, grads, bufs):
+            muon_update(_Matrices(ps), _Matrices(grads), _Matrices(bufs), **kw)
+            # as the copies back would: what saved a parameter sees that it changed
+            for t in (*ps, *bufs):
+                if not t.is_inference():
+                    torch.autograd.graph.increment_version(t)
+            return
         params = torch.stack([p.detach() for p in ps])
-        grads = torch.stack([p.grad.float() for p in ps])
+        grads = torch.stack([g.float() for g in grads])
         buf = torch.stack(bufs)
         muon_update(params, grads, buf, **kw)
         for i, p in enumerate(ps):
