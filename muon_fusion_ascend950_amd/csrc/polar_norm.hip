@@ -39,6 +39,27 @@ constexpr int kNormUnroll = 4;      // norm passes: 16 bytes per thread and iter
 constexpr int kMomentumUnroll = 2;  // momentum pass: 64 bytes per thread and iteration
 constexpr int kParamUnroll = 2;     // parameter pass: 48 bytes per thread and iteration
 
+// Element-wise loops (matrices of m·n % 8 != 0, whose sums run one element per thread
+// and step): loads issued ahead per thread, again in increasing order.  One at a time
+// each wave waited out every round trip: the Muon update of [20,127,2051] took 193 us,
+// that of [1,2047,4097] 574, the chain of [1,333,9999] 197; with these and the 16-byte
+// accesses below 180, 551 and 193.  (The padding copy keeps its 2-byte loads of odd rows:
+// unaligned 16-byte ones took it from 9.5 to 14.4 us at [1,333,9999].)
+constexpr int kElemUnroll = 8;
+
+// 16 bytes at any element's address: global memory takes unaligned vector accesses, at
+// the cost of a second line where one straddles it.
+template <typename V, typename T>
+__device__ __forceinline__ V load16_any(const T *p) {
+    V v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+template <typename V, typename T>
+__device__ __forceinline__ void store16_any(T *p, V v) {
+    __builtin_memcpy(p, &v, 16);
+}
+
 // Sum of v over the block in a fixed order: butterfly within each wave, then the
 // four wave totals in index order.  `red` holds 4 floats of LDS.
 __device__ __forceinline__ float block_sum(float v, float *red) {
@@ -77,9 +98,17 @@ __global__ __launch_bounds__(kNormThreads) void norm_partial_kernel(const uint16
             }
         }
     } else {
-        for (int64_t e = e0 + threadIdx.x; e < e1; e += kNormThreads) {
-            const float f = bf16_bits_to_f32(base[e]);
-            acc = fmaf(f, f, acc);
+        for (int64_t e = e0 + threadIdx.x; e < e1; e += kElemUnroll * kNormThreads) {
+            uint32_t v[kElemUnroll];
+#pragma unroll
+            for (int u = 0; u < kElemUnroll; ++u)
+                if (e + u * kNormThreads < e1) v[u] = base[e + u * kNormThreads];
+#pragma unroll
+            for (int u = 0; u < kElemUnroll; ++u) {
+                if (e + u * kNormThreads >= e1) break;
+                const float f = bf16_bits_to_f32(v[u]);
+                acc = fmaf(f, f, acc);
+            }
         }
     }
     const float t = block_sum(acc, red);
@@ -124,8 +153,22 @@ __global__ __launch_bounds__(kNormThreads) void norm_scale_kernel(const uint16_t
             }
         }
     } else {
-        for (int64_t e = e0 + threadIdx.x; e < e1; e += kNormThreads)
-            yb[e] = f32_to_bf16_bits(bf16_bits_to_f32(xb[e]) / d);
+        for (int64_t e = e0 + threadIdx.x * 8; e < e1; e += kNormStride) {
+            if (e + 8 <= e1) {
+                const u32x4 v = load16_any<u32x4>(xb + e);
+                u32x4 o;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const uint32_t lo = f32_to_bf16_bits(bf16_bits_to_f32(v[w] & 0xffffu) / d);
+                    const uint32_t hi = f32_to_bf16_bits(bf16_bits_to_f32(v[w] >> 16) / d);
+                    o[w] = lo | (hi << 16);
+                }
+                store16_any(yb + e, o);
+            } else {
+                for (int64_t i = e; i < e1; ++i)
+                    yb[i] = f32_to_bf16_bits(bf16_bits_to_f32(xb[i]) / d);
+            }
+        }
     }
 }
 
@@ -268,10 +311,23 @@ __global__ __launch_bounds__(kNormThreads) void muon_momentum_kernel(
             }
         }
     } else {
-        for (int64_t e = e0 + threadIdx.x; e < e1; e += kNormThreads) {
-            uint32_t h;
-            bufb[e] = one(grad_value(gb[e]), bufb[e], h);
-            x0[base + e] = static_cast<uint16_t>(h);
+        for (int64_t e = e0 + threadIdx.x; e < e1; e += kElemUnroll * kNormThreads) {
+            float gv[kElemUnroll], bv[kElemUnroll];
+#pragma unroll
+            for (int u = 0; u < kElemUnroll; ++u) {
+                const int64_t eu = e + u * kNormThreads;
+                if (eu >= e1) break;
+                gv[u] = grad_value(gb[eu]);
+                bv[u] = bufb[eu];
+            }
+#pragma unroll
+            for (int u = 0; u < kElemUnroll; ++u) {
+                const int64_t eu = e + u * kNormThreads;
+                if (eu >= e1) break;
+                uint32_t h;
+                bufb[eu] = one(gv[u], bv[u], h);
+                x0[base + eu] = static_cast<uint16_t>(h);
+            }
         }
     }
     const float t = block_sum(acc, red);
@@ -322,8 +378,23 @@ __global__ __launch_bounds__(kNormThreads) void muon_param_update_kernel(
     } else {
         for (int64_t e = (int64_t(blockIdx.x) * kNormThreads + threadIdx.x) * 8; e < total;
              e += stride) {
-            const int64_t end = e + 8 < total ? e + 8 : total;
-            for (int64_t i = e; i < end; ++i) p[i] = p[i] * decay + alpha * bf16_bits_to_f32(o[i]);
+            if (e + 8 <= total) {
+                const u32x4 ov = load16_any<u32x4>(o + e);
+                f32x4 q0 = load16_any<f32x4>(p + e), q1 = load16_any<f32x4>(p + e + 4);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    q0[2 * i] = q0[2 * i] * decay + alpha * bf16_bits_to_f32(ov[i] & 0xffffu);
+                    q0[2 * i + 1] = q0[2 * i + 1] * decay + alpha * bf16_bits_to_f32(ov[i] >> 16);
+                    q1[2 * i] = q1[2 * i] * decay + alpha * bf16_bits_to_f32(ov[i + 2] & 0xffffu);
+                    q1[2 * i + 1] =
+                        q1[2 * i + 1] * decay + alpha * bf16_bits_to_f32(ov[i + 2] >> 16);
+                }
+                store16_any(p + e, q0);
+                store16_any(p + e + 4, q1);
+            } else {
+                for (int64_t i = e; i < total; ++i)
+                    p[i] = p[i] * decay + alpha * bf16_bits_to_f32(o[i]);
+            }
         }
     }
 }
