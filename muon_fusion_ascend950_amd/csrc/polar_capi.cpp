@@ -53,20 +53,27 @@ uint64_t env_u64(const char *name, uint64_t def, bool *present = nullptr) {
     return end != v ? static_cast<uint64_t>(parsed) : def;
 }
 
-// Whether a MUON_POLAR_* variable that tunes the stage kernels is set (any but those that
-// leave them as they are).
-bool stage_knob_set() {
-    static const char *const kOthers[] = {"DEBUG_SYNC=", "CAPI_LIBRARY=", "RESIDENT="};
-    constexpr char kPrefix[] = "MUON_POLAR_";
+// Which MUON_POLAR_* variables are set, from one walk over the environment: any that
+// read_knobs reads, and any that tunes the stage kernels.  Nearly always none is, and the
+// walk stands for the two dozen look-ups of read_knobs, each a walk of its own.
+struct EnvSet {
+    bool any = false, stage = false;
+};
+EnvSet polar_env() {
+    constexpr char kPrefix[] = "MUON_POLAR_", kResident[] = "RESIDENT=";
+    static const char *const kOthers[] = {"DEBUG_SYNC=", "CAPI_LIBRARY="};
     constexpr size_t kLen = sizeof(kPrefix) - 1;
+    EnvSet set;
     for (char **e = environ; e != nullptr && *e != nullptr; ++e) {
         if (std::strncmp(*e, kPrefix, kLen) != 0) continue;
+        const char *name = *e + kLen;
         bool other = false;
-        for (const char *name : kOthers)
-            other = other || std::strncmp(*e + kLen, name, std::strlen(name)) == 0;
-        if (!other) return true;
+        for (const char *o : kOthers) other = other || std::strncmp(name, o, std::strlen(o)) == 0;
+        if (other) continue;
+        set.any = true;
+        if (std::strncmp(name, kResident, sizeof(kResident) - 1) != 0) set.stage = true;
     }
-    return false;
+    return set;
 }
 
 int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
@@ -278,21 +285,23 @@ int default_depth(int bm, int bn, int waves, int64_t tiles, int cus) {
 // X is [batch, m, n]; s = min(m, n) is the extent of A and P.
 int read_knobs(int64_t batch, int64_t m, int64_t n, int cus, Knobs &k) {
     const int64_t s = std::min(m, n);
-    k.waves = static_cast<uint32_t>(env_u64("MUON_POLAR_WAVES", kDefaultWaves));
+    const EnvSet set = polar_env();
+    auto env = [&](const char *name, uint64_t def) { return set.any ? env_u64(name, def) : def; };
+    k.waves = static_cast<uint32_t>(env("MUON_POLAR_WAVES", kDefaultWaves));
     if (k.waves != 4 && k.waves != 8)
         return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_WAVES must be 4 or 8");
-    k.resident = static_cast<uint32_t>(env_u64("MUON_POLAR_RESIDENT", 1));
+    k.resident = static_cast<uint32_t>(env("MUON_POLAR_RESIDENT", 1));
     if (k.resident > 1) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_RESIDENT must be 0 or 1");
-    if (stage_knob_set()) k.resident = 0;
-    k.pair = static_cast<uint32_t>(env_u64("MUON_POLAR_PAIR", 1));
+    if (set.stage) k.resident = 0;
+    k.pair = static_cast<uint32_t>(env("MUON_POLAR_PAIR", 1));
     if (k.pair > 1) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_PAIR must be 0 or 1");
-    k.halves = static_cast<uint32_t>(env_u64("MUON_POLAR_APPLY_HALVES", 1));
+    k.halves = static_cast<uint32_t>(env("MUON_POLAR_APPLY_HALVES", 1));
     if (k.halves > 2) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_APPLY_HALVES must be 0, 1 or 2");
     // three 48 KiB slots for the halves: [4096,14336] apply 395 -> 390 us
-    k.halves_depth = static_cast<uint32_t>(env_u64("MUON_POLAR_HALVES_DEPTH", 3));
-    k.diag_pairs = static_cast<uint32_t>(env_u64("MUON_POLAR_DIAG_PAIRS", 1));
+    k.halves_depth = static_cast<uint32_t>(env("MUON_POLAR_HALVES_DEPTH", 3));
+    k.diag_pairs = static_cast<uint32_t>(env("MUON_POLAR_DIAG_PAIRS", 1));
     if (k.diag_pairs > 1) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_DIAG_PAIRS must be 0 or 1");
-    k.sk_rounds = static_cast<uint32_t>(env_u64("MUON_POLAR_SK_ROUNDS", 7));
+    k.sk_rounds = static_cast<uint32_t>(env("MUON_POLAR_SK_ROUNDS", 7));
     if (k.sk_rounds > 7)
         return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_SK_ROUNDS must be a stage mask (0-7)");
     // Cache policy of the output stores: device-scope (sc1) stores of A, P and Y
@@ -304,13 +313,13 @@ int read_knobs(int64_t batch, int64_t m, int64_t n, int cus, Knobs &k) {
     // 37.9 -> 34.3, [2,2048,8192] 249.9 -> 244.1; single steps [8,512,2048] 34.7 ->
     // 34.2, [4096,14336] 671.7 -> 664.6 and 694.0 -> 690.9 (two boxes), [14336,4096]
     // 678.6 -> 672.5; [4,4096,4096] unchanged.
-    k.sk_share = static_cast<uint32_t>(env_u64("MUON_POLAR_SK_MIN_SHARE", 0));
+    k.sk_share = static_cast<uint32_t>(env("MUON_POLAR_SK_MIN_SHARE", 0));
     if (k.sk_share > 4096) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_SK_MIN_SHARE must be 0..4096");
-    k.sk_pieces = static_cast<uint32_t>(env_u64("MUON_POLAR_SK_PIECES", 0));
+    k.sk_pieces = static_cast<uint32_t>(env("MUON_POLAR_SK_PIECES", 0));
     if (k.sk_pieces == 1 || k.sk_pieces > 16)
         return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_SK_PIECES must be 0 (by tile) or 2..16");
-    k.y_cpol = static_cast<uint32_t>(env_u64("MUON_POLAR_Y_CPOL", 2));
-    k.ap_cpol = static_cast<uint32_t>(env_u64("MUON_POLAR_AP_CPOL", 2));
+    k.y_cpol = static_cast<uint32_t>(env("MUON_POLAR_Y_CPOL", 2));
+    k.ap_cpol = static_cast<uint32_t>(env("MUON_POLAR_AP_CPOL", 2));
     if (k.y_cpol > 4 || k.ap_cpol > 4)
         return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_Y_CPOL / _AP_CPOL must be 0..4");
     if (k.halves_depth != 2 && k.halves_depth != 3)
@@ -341,28 +350,28 @@ int read_knobs(int64_t batch, int64_t m, int64_t n, int cus, Knobs &k) {
     }
     if (gram_tile == 256 && k.waves == 8 && k.pair == 1 && one_round_of_192(batch, s, cus))
         gram_tile = 192;
-    k.gram_tile = static_cast<uint32_t>(env_u64("MUON_POLAR_GRAM_TILE", gram_tile));
+    k.gram_tile = static_cast<uint32_t>(env("MUON_POLAR_GRAM_TILE", gram_tile));
     // an explicit gram tile also sets the poly tile unless that is given too
-    const bool gram_set = std::getenv("MUON_POLAR_GRAM_TILE") != nullptr;
+    const bool gram_set = set.any && std::getenv("MUON_POLAR_GRAM_TILE") != nullptr;
     uint32_t poly_tile = default_sym_tile(batch, s, 4096, cus);
     if (poly_tile == 256 && one_round_of_192(batch, s, cus)) poly_tile = 192;
     k.poly_tile = static_cast<uint32_t>(
-        env_u64("MUON_POLAR_POLY_TILE", gram_set ? k.gram_tile : poly_tile));
+        env("MUON_POLAR_POLY_TILE", gram_set ? k.gram_tile : poly_tile));
     k.apply_bm = static_cast<uint32_t>(
-        env_u64("MUON_POLAR_APPLY_TILE_M", default_apply_tile(batch, m, n, cus)));
-    k.apply_bn = static_cast<uint32_t>(env_u64("MUON_POLAR_APPLY_TILE_N", k.apply_bm));
-    k.stream = static_cast<uint32_t>(env_u64("MUON_POLAR_STREAM", 1));
+        env("MUON_POLAR_APPLY_TILE_M", default_apply_tile(batch, m, n, cus)));
+    k.apply_bn = static_cast<uint32_t>(env("MUON_POLAR_APPLY_TILE_N", k.apply_bm));
+    k.stream = static_cast<uint32_t>(env("MUON_POLAR_STREAM", 1));
     if (k.stream > 1) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_STREAM must be 0 or 1");
     // MUON_POLAR_STREAM_K: 0 off, 1 on (every stage); MUON_POLAR_STREAM_K_STAGES
     // narrows it to a stage mask (bit 0 gram, bit 1 poly, bit 2 apply).
-    k.stream_k = static_cast<uint32_t>(env_u64("MUON_POLAR_STREAM_K", 1));
+    k.stream_k = static_cast<uint32_t>(env("MUON_POLAR_STREAM_K", 1));
     if (k.stream_k > 1) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_STREAM_K must be 0 or 1");
-    const uint64_t sk_stages = env_u64("MUON_POLAR_STREAM_K_STAGES", 7);
+    const uint64_t sk_stages = env("MUON_POLAR_STREAM_K_STAGES", 7);
     if (sk_stages > 7) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_STREAM_K_STAGES must be 0..7");
     k.stream_k *= static_cast<uint32_t>(sk_stages);
-    k.depth[0] = static_cast<uint32_t>(env_u64("MUON_POLAR_GRAM_DEPTH", 0));
-    k.depth[1] = static_cast<uint32_t>(env_u64("MUON_POLAR_POLY_DEPTH", 0));
-    k.depth[2] = static_cast<uint32_t>(env_u64("MUON_POLAR_APPLY_DEPTH", 0));
+    k.depth[0] = static_cast<uint32_t>(env("MUON_POLAR_GRAM_DEPTH", 0));
+    k.depth[1] = static_cast<uint32_t>(env("MUON_POLAR_POLY_DEPTH", 0));
+    k.depth[2] = static_cast<uint32_t>(env("MUON_POLAR_APPLY_DEPTH", 0));
     for (uint32_t d : k.depth)
         if (d > 8) return fail(MUON_POLAR_ERR_CONFIG, "MUON_POLAR_*_DEPTH must be 0 (auto) or 2..8");
     if (!muon_polar::tile_supported(Stage::Gram, k.gram_tile, k.gram_tile))
