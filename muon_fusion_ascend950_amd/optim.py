@@ -60,7 +60,8 @@ def _updatable_in_place(params, grads, bufs) -> bool:
     ordinary contiguous GPU tensors of one shape, gradients of one dtype, and nothing
     that is written shares memory with another tensor.  A tall matrix whose width is no
     multiple of 8 has no native form (its update runs on the transposed matrix), and
-    traced programs keep to the operations on tensors."""
+    traced programs and tensors that a function transform wraps (which have no address)
+    keep to the operations on tensors."""
     shape, device, dtype = params[0].shape, params[0].device, grads[0].dtype
     if (torch.compiler.is_compiling() or device.type != "cuda" or len(shape) < 2
             or 0 in shape or dtype not in (torch.float32, torch.bfloat16)
@@ -74,7 +75,10 @@ def _updatable_in_place(params, grads, bufs) -> bool:
                     or t.shape != shape or t.device != device or not t.is_contiguous()
                     or t.is_neg()):
                 return False
-            start = t.data_ptr()
+            try:
+                start = t.data_ptr()
+            except RuntimeError:
+                return False
             ranges.append((start, start + t.numel() * t.element_size(), written))
     ranges.sort()
     end_any = end_written = 0

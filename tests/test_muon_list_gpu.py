@@ -106,3 +106,28 @@ def test_step_of_apart_parameters_is_seen_by_autograd():
     Muon(params, lr=0.1).step()
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         y.backward()
+
+
+@pytest.mark.parametrize("transform", ["grad", "jvp"])
+def test_a_bfloat16_gradient_inside_a_function_transform(transform):
+    """The transforms wrap what is computed from their input in tensors without an
+    address; the update takes those too, through the operations on tensors."""
+    import muon_fusion_ascend950_amd.optim as optim
+
+    gen = torch.Generator(device=DEV).manual_seed(7)
+    (p,), (x,), (b,) = (tensors(1, (2, 32, 48), gen) for _ in range(3))
+    want_p, want_b = p.clone(), b.clone()
+    optim.muon_update(want_p, (2 * x).bfloat16(), want_b, **KW)
+
+    def f(x):
+        q, buf = p + 0 * x.detach(), b + 0 * x.detach()
+        optim.muon_update(q, (2 * x.detach()).bfloat16(), buf, **KW)
+        return (x * x).sum(), (q, buf)
+
+    if transform == "grad":
+        d, (q, buf) = torch.func.grad(f, has_aux=True)(x)
+        assert torch.equal(d, 2 * x)
+    else:
+        _, d, (q, buf) = torch.func.jvp(f, (x,), (torch.ones_like(x),), has_aux=True)
+        assert torch.allclose(d, 2 * x.sum(), rtol=1e-4)
+    assert torch.equal(q, want_p) and torch.equal(buf, want_b)
