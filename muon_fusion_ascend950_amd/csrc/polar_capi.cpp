@@ -20,7 +20,9 @@
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <numeric>
 #include <string>
 #include <unordered_map>
@@ -1277,11 +1279,14 @@ int update_tensors(const muon_polar::MuonTensors &t, void *workspace, size_t wor
     };
     const uintptr_t f32_bytes = static_cast<uintptr_t>(t.matrices * m * n * 4);
     const uintptr_t g_bytes = t.grad_bf16 ? f32_bytes / 2 : f32_bytes;
-    std::vector<Range> ranges;
-    ranges.reserve(static_cast<size_t>(3 * t.count + 1));
+    // (no exception may leave a C entry point)
+    const std::unique_ptr<Range[]> ranges(new (std::nothrow) Range[3 * t.count + 1]);
+    if (ranges == nullptr)
+        return fail(MUON_POLAR_ERR_INVALID_ARGUMENT, "out of host memory for this many tensors");
+    Range *end = ranges.get();
     auto add = [&](const void *q, uintptr_t bytes, bool written) {
         const uintptr_t lo = reinterpret_cast<uintptr_t>(q);
-        ranges.push_back({lo, lo + bytes, written});
+        *end++ = {lo, lo + bytes, written};
     };
     add(workspace, static_cast<uintptr_t>(p.muon_workspace_bytes), true);
     bool vec_gb = true, vec_p = true;
@@ -1292,10 +1297,10 @@ int update_tensors(const muon_polar::MuonTensors &t, void *workspace, size_t wor
         vec_gb = vec_gb && aligned16(t.grad[i]) && aligned16(t.buf[i]);
         vec_p = vec_p && aligned16(t.param[i]);
     }
-    std::sort(ranges.begin(), ranges.end(),
-              [](const Range &x, const Range &y) { return x.lo < y.lo; });
+    std::sort(ranges.get(), end, [](const Range &x, const Range &y) { return x.lo < y.lo; });
     uintptr_t end_any = 0, end_written = 0;
-    for (const Range &r : ranges) {
+    for (const Range *q = ranges.get(); q != end; ++q) {
+        const Range &r = *q;
         if (r.lo < (r.written ? end_any : end_written))
             return fail(MUON_POLAR_ERR_INVALID_ARGUMENT,
                         "param, grad, momentum_buffer and workspace must not overlap");

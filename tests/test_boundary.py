@@ -429,3 +429,31 @@ def test_stage_calls_reject_overlapping_buffers_before_any_launch():
     ews = info.express_workspace_bytes
     assert lib.muon_polar_express(X, W + 4096, W, ews, batch, m, n, coeffs, 1, 1, None) == bad
     assert "workspace must not overlap" in capi.last_error()
+
+
+def test_update_list_out_of_host_memory_is_an_error_code():
+    """2^20 tensors need 72 MiB to look for overlaps: where they cannot be had, the C entry
+    returns an error and throws nothing (a process of its own, its address space limited;
+    one address for all tensors, so that no call gets as far as a launch)."""
+    code = """
+import ctypes, resource
+import numpy as np
+from muon_fusion_ascend950_amd import capi
+lib = capi.load()
+count = 1 << 20
+addr = np.full(count, 1 << 40, dtype=np.uint64).ctypes.data_as(ctypes.POINTER(ctypes.c_void_p))
+coef = (ctypes.c_double * 3)(1, 1, 1)
+def call(n):
+    st = lib.muon_polar_muon_update_list(addr, addr, 0, addr, n, 1 << 41, 1 << 45, 1, 8, 8, 0.9, 1,
+                                         coef, 1, 0.1, 0.0, 1.0, None)
+    print(st, capi.last_error(), flush=True)
+call(2)
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (32 << 20),) * 2)
+call(count)
+"""
+    proc = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT)
+    assert proc.returncode == 0, proc.stderr
+    first, second = proc.stdout.strip().splitlines()[-2:]
+    assert first.startswith("-1 ") and "overlap" in first
+    assert second.startswith("-1 ") and "out of host memory" in second
