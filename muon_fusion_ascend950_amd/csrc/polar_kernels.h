@@ -146,8 +146,8 @@ struct MuonTensors {
     bool grad_bf16;
 };
 
-// Matrices (momentum pass) or tensors (parameter pass) of one launch whose pointers
-// travel in its arguments: 2 KiB of the 4 KiB that a launch takes.
+// Tensors of one launch of the momentum or parameter pass, whose pointers travel in its
+// arguments: 2 KiB of the 4 KiB that a launch takes.
 constexpr int kMuonListMax = 128;
 
 // Muon update passes (polar_norm.hip).  Momentum: buf ← lerp(buf, g, w),

@@ -4,6 +4,8 @@ takes (128 matrices) and of the element paths (vector, 8 at a time, one at a tim
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -131,3 +133,41 @@ def test_a_bfloat16_gradient_inside_a_function_transform(transform):
         _, d, (q, buf) = torch.func.jvp(f, (x,), (torch.ones_like(x),), has_aux=True)
         assert torch.allclose(d, 2 * x.sum(), rtol=1e-4)
     assert torch.equal(q, want_p) and torch.equal(buf, want_b)
+
+
+def graph_nodes(f):
+    """Nodes (launches) of `f` captured in a graph."""
+    f()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        f()
+    with open("/proc/self/maps") as maps:
+        path = next(line.split()[-1] for line in maps if "libamdhip64.so" in line)
+    nodes = ctypes.c_size_t(0)
+    assert ctypes.CDLL(path).hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None,
+                                              ctypes.byref(nodes)) == 0
+    return nodes.value
+
+
+@pytest.mark.parametrize("count,shape,launches", [
+    (4, (300, 16, 24), 1),  # several matrices in each tensor: one pointer per tensor
+    (129, (3, 16, 24), 2),
+])
+def test_launches_of_a_pass_follow_the_tensors_not_their_matrices(monkeypatch, count, shape,
+                                                                  launches):
+    import muon_fusion_ascend950_amd.optim as optim
+
+    monkeypatch.delenv("MUON_POLAR_RESIDENT", raising=False)
+    gen = torch.Generator(device=DEV).manual_seed(count)
+    p, g, b = (tensors(count, shape, gen) for _ in range(3))
+    sp, sg, sb = torch.stack(p), torch.stack(g), torch.stack(b)
+    apart = [optim._Matrices(t) for t in (p, g, b)]
+    update = lambda: optim.muon_update(*apart, **KW)
+    # the iteration, and the momentum and the parameter pass
+    assert graph_nodes(update) == 1 + 2 * launches
+    for t, s in ((p, sp), (b, sb)):
+        for i, u in enumerate(t):
+            u.copy_(s[i])
+    update()
+    optim.muon_update(sp, sg, sb, **KW)
+    assert torch.equal(torch.stack(p), sp) and torch.equal(torch.stack(b), sb)
