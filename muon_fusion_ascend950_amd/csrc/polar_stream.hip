@@ -230,6 +230,11 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     int tid = static_cast<int>(threadIdx.x);
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63;
+    // Row and first column, within the wave tile, of this lane's group q of block (i, j)
+    auto grp_r = [&](int i) { return i * kB + (lane & (kB - 1)); };
+    auto grp_c = [&](int j, int q) {
+        return k16 ? 16 * j + 4 * (lane >> 4) : 32 * j + 8 * q + 4 * (lane >> 5);
+    };
     // Swizzles of the K- and N-contiguous panels
     auto kcs = [&](int row) { return k16 ? kc_swz16(row) : kc_swz(row); };
     auto ncs = [&](auto bn_c, int krow) {
@@ -343,22 +348,13 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
         return off;
     };
     auto dma_one = [&](int d, int step, int slot, bool live) {
-        // (written out: through a_voff and b_voff the K-masked 64x64 gram took 18 more
-        // scalar reloads and 33 more wait states)
-        const int k0 = step * kBK;
         if (d < Geo::kLoadsA) {
-            const uint32_t koff = live ? a_step(k0) : kOob;
-            uint32_t off = off_a[d] + koff;
-            if constexpr (KT) off = k0 + 8 * a_chunk(d) < g.row_k ? off : kOob;
             const uint32_t dst = smem_base + slot_a(slot) + (wave * Geo::kLoadsA + d) * 1024;
-            dma_16B(rs_row, live ? dst : sink_base, off);
+            dma_16B(rs_row, live ? dst : sink_base, a_voff(d, step, live));
         } else {
             const int i = d - Geo::kLoadsA;
-            const uint32_t koff = live ? b_step(k0) : kOob;
-            uint32_t off = off_b[i] + koff;
-            if constexpr (KT) off = k0 + 8 * b_chunk(i) < g.col_k ? off : kOob;
             const uint32_t dst = smem_base + slot_b(slot) + (wave * Geo::kLoadsB + i) * 1024;
-            dma_16B(rs_col, live ? dst : sink_base, off);
+            dma_16B(rs_col, live ? dst : sink_base, b_voff(i, step, live));
         }
     };
     // KT with rows of n % 8 != 0 elements (gram reading X rows of even length in
@@ -390,17 +386,15 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
             // live in scalar registers and spill)
             int wv = wave;
             asm volatile("" : "+s"(wv));
-            const uint32_t base = smem_base + ao + 16 * lane;
-            const uint32_t to_b = Geo::kPanelRing ? bo - ao : Geo::kABytes;
 #pragma unroll
             for (int d = 0; d < Geo::kLoads; ++d) {
-                const uint32_t dst =
-                    d < Geo::kLoadsA
-                        ? base + (wv * Geo::kLoadsA + d) * 1024
-                        : base + to_b + (wv * Geo::kLoadsB + d - Geo::kLoadsA) * 1024;
+                const int dst = (d < Geo::kLoadsA
+                                     ? ao + (wv * Geo::kLoadsA + d) * 1024
+                                     : bo + (wv * Geo::kLoadsB + d - Geo::kLoadsA) * 1024) +
+                                16 * lane;
                 // keep values 0 .. rem-1 of the chunk (all of it when rem is 0)
                 const int rem = static_cast<int>((tail_rem >> (4 * d)) & 15u);
-                u32x4 *q = reinterpret_cast<u32x4 *>(smem + (dst - smem_base) / 2);
+                u32x4 *q = reinterpret_cast<u32x4 *>(smem + dst / 2);
                 u32x4 v = *q;
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
@@ -472,7 +466,7 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     }
     auto load_frag = [&](int ao, int bo, int kk, int f, bf16x8 (&fr)[SM], bf16x8 (&fc)[SN]) {
         const uint16_t *as = smem + ao / 2;
-        const uint16_t *bs = as + Geo::kABytes / 2;  // (the 32x32x16 kernels: slots, not panels)
+        const uint16_t *bs = smem + bo / 2;
         if constexpr (k16) {  // kk: k32 slice
             // (`lane` parts opaque here: their combinations with the fragment's uniform part
             // would otherwise all be formed outside the K loop and spill)
@@ -524,14 +518,16 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     auto add_ax = [&](int ao, int bo, int kg) {
         if constexpr (kAxInLoop) {
             if (!acc_owner) return;  // wave pairs: a·X goes into the h = 0 half once
-            // the large tiles: an opaque copy of the lane index keeps the address
-            // arithmetic in the few steps that use it (hoisted out of the K loop it
-            // would spill)
+            // an opaque copy of the lane index keeps the address arithmetic in the few
+            // steps that use it (hoisted out of the K loop it would spill)
             int ln = lane;
-            if constexpr (k16) asm volatile("" : "+v"(ln));
-            constexpr int kLog = k16 ? 4 : 5;  // a lane's row ln mod kB, first column 4 (ln / kB)
+            asm volatile("" : "+v"(ln));
+            const int lane_r = ln & (kB - 1);
+            auto lane_c = [&](int j, int q) {
+                return k16 ? 16 * j + 4 * (ln >> 4) : 32 * j + 8 * q + 4 * (ln >> 5);
+            };
             const uint16_t *as = smem + ao / 2;
-            const uint16_t *bs = kPanelRing ? smem + bo / 2 : as + Geo::kABytes / 2;
+            const uint16_t *bs = smem + bo / 2;
             const float a = g.s_epi;
             auto fma4 = [&](AccT &acc_ij, int q, u32x2 v) {
                 float x[4];
@@ -542,53 +538,51 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
             if constexpr (S == Stage::Apply) {
                 const int rel = kg * kBK - row0;  // tile row of the step's first K-row
                 if (rel < 0 || rel >= BM) return;
-                auto add_rows = [&](int i, int kr) {
-#pragma unroll
-                    for (int j = 0; j < SN; ++j)
-#pragma unroll
-                        for (int q = 0; q < kNQ; ++q) {
-                            const int c = wc * WN + kB * j + 8 * q + 4 * (ln >> kLog);
-                            int at;
-                            if constexpr (k16)
-                                at = nc_offset16<BN>(kr, c >> 3);
-                            else
-                                at = nc_offset<BN>(kr, c >> 3);
-                            fma4(acc[i][j], q,
-                                 *reinterpret_cast<const u32x2 *>(bs + at + (c & 7)));
-                        }
-                };
-                // large tiles: row blocks that fit a K-step share one branch
-                constexpr int kGrp = k16 && WM >= kBK ? kBK / kB : 1;
+                // row blocks that fit a K-step share one branch
+                constexpr int kGrp = WM >= kBK ? kBK / kB : 1;
 #pragma unroll
                 for (int i0 = 0; i0 < SM; i0 += kGrp) {
                     const int rb = wr * WM + kB * i0;
                     if (rb < rel || rb >= rel + kBK) continue;
 #pragma unroll
-                    for (int i = 0; i < kGrp; ++i) add_rows(i0 + i, rb - rel + (ln & (kB - 1)) + kB * i);
+                    for (int i = i0; i < i0 + kGrp; ++i) {
+                        const int kr = rb + kB * (i - i0) - rel + lane_r;
+#pragma unroll
+                        for (int j = 0; j < SN; ++j)
+#pragma unroll
+                            for (int q = 0; q < kNQ; ++q) {
+                                const int c = wc * WN + lane_c(j, q);
+                                const int pos =
+                                    (c >> 3) ^ ncs(std::integral_constant<int, BN>{}, kr);
+                                fma4(acc[i][j], q,
+                                     *reinterpret_cast<const u32x2 *>(bs + kr * BN + 8 * pos +
+                                                                      (c & 7)));
+                            }
+                    }
                 }
             } else {
                 const int rel = kg * kBK - col0;  // tile column of the step's first K
                 if (rel < 0 || rel >= BN) return;
-                auto add_cols = [&](int j, int cb) {
-#pragma unroll
-                    for (int i = 0; i < SM; ++i) {
-                        const int r = wr * WM + kB * i + (ln & (kB - 1));
-#pragma unroll
-                        for (int q = 0; q < kNQ; ++q) {
-                            const int kc = cb + 8 * q + 4 * (ln >> kLog);
-                            const int at = k16 ? kc_offset16(r, kc >> 3) : kc_offset(r, kc >> 3);
-                            fma4(acc[i][j], q,
-                                 *reinterpret_cast<const u32x2 *>(as + at + (kc & 7)));
-                        }
-                    }
-                };
-                constexpr int kGrp = k16 && WN >= kBK ? kBK / kB : 1;
+                constexpr int kGrp = WN >= kBK ? kBK / kB : 1;
 #pragma unroll
                 for (int j0 = 0; j0 < SN; j0 += kGrp) {
                     const int cb = wc * WN + kB * j0;
                     if (cb < rel || cb >= rel + kBK) continue;
 #pragma unroll
-                    for (int j = 0; j < kGrp; ++j) add_cols(j0 + j, cb - rel + kB * j);
+                    for (int j = j0; j < j0 + kGrp; ++j) {
+#pragma unroll
+                        for (int i = 0; i < SM; ++i) {
+                            const int r = wr * WM + kB * i + lane_r;
+#pragma unroll
+                            for (int q = 0; q < kNQ; ++q) {
+                                const int kc = wc * WN + lane_c(j, q) - rel;
+                                fma4(acc[i][j], q,
+                                     *reinterpret_cast<const u32x2 *>(
+                                         as + r * kBK + (((kc >> 3) ^ kcs(r)) << 3) +
+                                         (kc & 7)));
+                            }
+                        }
+                    }
                 }
             }
         }
@@ -1225,15 +1219,15 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     if (acc_owner) {
 #pragma unroll
         for (int i = 0; i < SM; ++i) {
-            const int r = wr * WM + i * kB + (lane & (kB - 1));
+            const int r = wr * WM + grp_r(i);
 #pragma unroll
             for (int j = 0; j < SN; ++j) {
 #pragma unroll
                 for (int q = 0; q < kNQ; ++q) {
                     // diagonal pairs: block (h,h), and (0,1) for h = 0
                     if (DG && hr == 1 && j == 1) continue;
-                    const int cb = DG ? (j == 0 ? 32 * hr : 32) : wc * WN + j * kB;
-                    const int c = cb + (k16 ? 4 * (lane >> 4) : 8 * q + 4 * (lane >> 5));
+                    const int c = DG ? (j == 0 ? 32 * hr : 32) + 8 * q + 4 * (lane >> 5)
+                                     : wc * WN + grp_c(j, q);
                     u32x2 *p = reinterpret_cast<u32x2 *>(at(dt, r, c));
                     float e[4] = {0.f, 0.f, 0.f, 0.f};
                     uint16_t h[4];
