@@ -256,6 +256,8 @@ typedef struct muon_polar_plan_extents {
        steps before the last, which writes its iterate padded to np columns (out_limit:
        the padded buffer); all zero for other shapes. */
     muon_polar_stage_extent chain_apply;
+    int32_t resident;  /* whole steps in one workgroup per matrix instead of the stages above:
+                          bit 0 single steps, bit 1 chains (polar_express, the Muon update) */
 } muon_polar_plan_extents;
 
 int muon_polar_check_plan(int64_t batch, int64_t m, int64_t n, int cus, const int *blocks_per_cu,

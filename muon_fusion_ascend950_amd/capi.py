@@ -57,7 +57,8 @@ class PlanExtents(ctypes.Structure):
     _fields_ = [(name, ctypes.c_int64) for name in (
         "workspace_bytes", "gram_bytes", "poly_offset", "counters_offset", "counter_stride",
         "partials_offset", "pad_offset", "pad_end", "y_bytes")] + [
-        ("stage", StageExtent * 3), ("chain_apply", StageExtent)]
+        ("stage", StageExtent * 3), ("chain_apply", StageExtent),
+        ("resident", ctypes.c_int32)]
 
 
 class CapiError(RuntimeError):

@@ -172,7 +172,8 @@ struct Plan {
     int64_t gram_grid, poly_grid, apply_grid;
     size_t gram_bytes, workspace_bytes;
     bool stream;
-    bool resident;  // steps run in polar_resident.hip's kernel (the stage calls never do)
+    // single steps / chains run in polar_resident.hip's kernel (the stage calls never do)
+    bool resident, resident_chain;
     int y_cpol, ap_cpol;  // store cache policies (GemmArgs::out_cpol)
     int waves[3];  // waves per workgroup of the DMA-fed kernel of each stage
     int depth[3];  // LDS ring slots of the DMA-fed kernel of each stage
@@ -512,9 +513,18 @@ constexpr int64_t kMaxMatrixElems = int64_t(1) << 30;
 // against stages: [64,64] 5.4 / 12.5 us, [129,130] 12.2 / 15.8, [3,129,257] 17.2 / 18.1,
 // [128,384] 13.6 / 14.3, left to the stages [128,480] 15.4 / 15.1, [150,271] 18.3 / 17.6,
 // tall [384,128] 17.4 / 14.0.  From 64 matrices on the stages' tiles add up ([64,192,192]
-// 17.0 / 19.1, [300,160,256] 31 / 66, [600,96,400] 39 / 92).  A single step decides, not a
-// chain (which gains more): both take one route, so a chain's results are its steps'.
-bool resident_pays(int64_t batch, int64_t m, int64_t n) {
+// 17.0 / 19.1, [300,160,256] 31 / 66, [600,96,400] 39 / 92).  From 256 on the resident kernel
+// is the faster one for every shape that fits, in one round of the CUs or more (60 shapes at
+// 255 to 1025 matrices: [257,480,128] 40 / 59, [257,31,1018] 22 / 65).
+// A single step decides, not a chain (which gains more): both take one route, so a chain's
+// results are its steps'.  One exception: tall matrices of four row blocks, 64 to 85 of them,
+// whose three gram tiles each are one round of the CUs.  Their steps end even at 1700
+// (counting the transposed columns' scattering once more by half where n % 32 != 0):
+// [64,320,128] 16.7 / 17.3, [64,352,128] 17.5 / 17.7, but [64,384,128] 18.6 / 17.8,
+// [64,320,120] 17.9 / 17.6, [64,448,120] 22.4 / 18.1; their chains of five steps gain all the
+// same ([64,384,128] 56 / 97 us).  There the stages are neither split nor paired, so steps and
+// chains have the same bits on either route.
+bool resident_pays(int64_t batch, int64_t m, int64_t n, bool chain) {
     if (muon_polar::resident_fit(m, n) == 0) return false;
     if (batch >= 256) return true;
     static constexpr int kBase[muon_polar::kResidentBlocks + 1] = {0, 150, 170, 320, 300, 410, 520};
@@ -524,7 +534,10 @@ bool resident_pays(int64_t batch, int64_t m, int64_t n) {
     const int64_t cost =
         kBase[nb] + kSlope[nb] * lb + (scattered ? 350 + m * n / 100 : 360);
     const int64_t stages = m > n ? 1380 : n % 8 == 0 ? 1440 : n % 2 == 0 ? 1640 : 1780;
-    return cost <= (batch >= 64 ? 2000 : stages);
+    if (batch < 64) return cost <= stages;
+    if (!chain && m > n && nb == 4 && 3 * batch <= 256)
+        return cost + (n % 32 != 0 ? m * n / 200 : 0) <= 1700;
+    return cost <= 2000;
 }
 
 int build_plan(int64_t batch, int64_t m, int64_t n, const Knobs &knobs, const Target &tgt,
@@ -557,7 +570,8 @@ int build_plan(int64_t batch, int64_t m, int64_t n, const Knobs &knobs, const Ta
     // The right-Gram stages exist only as DMA-fed kernels: MUON_POLAR_STREAM=0
     // selects the register-staged kernels for m <= n alone.
     p.stream = knobs.stream != 0 || tall;
-    p.resident = knobs.resident != 0 && resident_pays(batch, m, n);
+    p.resident = knobs.resident != 0 && resident_pays(batch, m, n, false);
+    p.resident_chain = knobs.resident != 0 && resident_pays(batch, m, n, true);
     p.y_cpol = static_cast<int>(knobs.y_cpol);
     p.ap_cpol = static_cast<int>(knobs.ap_cpol);
     if (p.gram_grid >= (int64_t(1) << 31) || p.apply_grid >= (int64_t(1) << 31))
@@ -1154,7 +1168,8 @@ int pad_input(const Plan &p, void *workspace, const void *x, int64_t batch, hipS
 // Whether the plan runs `steps` steps (after the normalisation, if asked) in one launch
 // of the resident kernel.
 bool resident_runs(const Plan &p, int64_t batch, int64_t steps, bool normalize) {
-    return p.resident && steps >= 1 && steps <= muon_polar::kResidentSteps &&
+    return (steps == 1 && !normalize ? p.resident : p.resident_chain) && steps >= 1 &&
+           steps <= muon_polar::kResidentSteps &&
            (!normalize || muon_polar::norm_chunk(batch, p.m * p.n) == 4096);
 }
 
@@ -1825,6 +1840,7 @@ int muon_polar_check_plan(int64_t batch, int64_t m, int64_t n, int cus, const in
     out->pad_offset = static_cast<int64_t>(p.pad_offset);
     out->pad_end = p.pad ? static_cast<int64_t>(p.pad_offset) + batch * m * p.np * 2 : 0;
     out->y_bytes = batch * m * n * 2;
+    out->resident = (p.resident ? 1 : 0) | (p.resident_chain ? 2 : 0);
     // The step's route on stand-in addresses (16-byte aligned, never dereferenced):
     // the workspace, X and Y in address ranges of their own.
     char *ws = reinterpret_cast<char *>(uintptr_t(1) << 44);

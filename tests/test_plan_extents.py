@@ -14,6 +14,8 @@ over 1-4 per stage, which covers what the device reports for every kernel.
 
 from __future__ import annotations
 
+import os
+
 import pytest
 
 from muon_fusion_ascend950_amd import capi
@@ -368,3 +370,32 @@ def test_apply_short_last_round_splits_with_the_round_before(shape, rem):
     assert e.halves == 0 and (e.tile_m, e.tile_n) == (256, 256)
     assert e.total_tiles % 256 == rem
     assert e.dp_tiles == e.total_tiles - rem - 256 and e.sk_units == 256
+
+
+@pytest.mark.parametrize("shape,resident", [
+    ((1, 64, 64), 3), ((1, 129, 130), 3), ((3, 129, 257), 3), ((1, 128, 384), 3),
+    ((1, 128, 480), 0), ((1, 384, 128), 0), ((63, 384, 128), 0),
+    # tall with four row blocks, one round of gram tiles: single steps are faster in stages
+    ((64, 384, 128), 2), ((64, 448, 120), 2), ((85, 352, 120), 2), ((64, 320, 120), 2),
+    ((64, 256, 128), 3), ((64, 288, 104), 3), ((85, 352, 128), 3),
+    # more than a round
+    ((86, 384, 128), 3), ((86, 448, 120), 3), ((192, 384, 104), 3),
+    # other tall shapes, and wide ones, from 64 matrices
+    ((64, 640, 96), 3), ((64, 288, 160), 3), ((64, 768, 64), 3), ((64, 192, 192), 3),
+    ((255, 480, 128), 0), ((256, 480, 128), 3), ((257, 480, 128), 3), ((256, 256, 192), 0),
+])
+def test_the_resident_route_is_the_measured_one(monkeypatch, shape, resident):
+    """Which steps (1) and chains (2) run in one workgroup per matrix, at the sides of each
+    measured line; where the two differ, the stages run each sum whole and in order."""
+    for k in [k for k in os.environ if k.startswith("MUON_POLAR_") and k != "MUON_POLAR_CAPI_LIBRARY"]:
+        monkeypatch.delenv(k)
+    plan = lambda: capi.check_plan(*shape, cus=256, blocks_per_cu=(2, 2, 2))
+    route = lambda: plan().resident
+    assert route() == resident
+    if resident == 2:
+        assert all(e.sk_units == 0 and e.diag_pairs == 0 for e in plan().stage)
+    monkeypatch.setenv("MUON_POLAR_RESIDENT", "0")
+    assert route() == 0
+    monkeypatch.delenv("MUON_POLAR_RESIDENT")
+    monkeypatch.setenv("MUON_POLAR_STREAM_K", "1")  # any tuning variable of the stages
+    assert route() == 0

@@ -6,6 +6,8 @@ a chain of any length."""
 
 from __future__ import annotations
 
+import os
+
 import pytest
 import torch
 
@@ -81,3 +83,14 @@ def test_infinities_and_nans_stay_in_their_matrix(mf):
     y = mf.polar_step(bad, *O.COEFFICIENTS[0])
     assert torch.equal(y[0], clean[0]) and torch.equal(y[2], clean[2])
     assert not torch.isfinite(y[1].float()).any()
+
+
+@pytest.mark.parametrize("shape", [(64, 384, 128), (85, 352, 120)])
+def test_a_chain_is_its_steps_where_only_the_chain_is_resident(monkeypatch, mf, shape):
+    for k in [k for k in os.environ if k.startswith("MUON_POLAR_") and k != "MUON_POLAR_CAPI_LIBRARY"]:
+        monkeypatch.delenv(k)
+    x = O.make_input(shape, seed=64).to(DEV)
+    want = x
+    for c in O.COEFFICIENTS:
+        want = mf.polar_step(want, *c)
+    assert torch.equal(mf.polar_express(x, O.COEFFICIENTS, normalize=False), want)
