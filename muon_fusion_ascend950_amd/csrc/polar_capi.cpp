@@ -1165,29 +1165,42 @@ int pad_input(const Plan &p, void *workspace, const void *x, int64_t batch, hipS
     return MUON_POLAR_OK;
 }
 
-// Whether the plan runs `steps` steps (after the normalisation, if asked) in one launch
-// of the resident kernel.
-bool resident_runs(const Plan &p, int64_t batch, int64_t steps, bool normalize) {
-    return (steps == 1 && !normalize ? p.resident : p.resident_chain) && steps >= 1 &&
-           steps <= muon_polar::kResidentSteps &&
-           (!normalize || muon_polar::norm_chunk(batch, p.m * p.n) == 4096);
+// Whether a chain of `steps` steps (after the normalisation, if asked) runs in the resident
+// kernel.  A single step's own route is a chain's too, except as resident_pays says.
+bool resident_runs(const Plan &p, int64_t steps, bool normalize) {
+    return steps >= 1 && (steps == 1 && !normalize ? p.resident : p.resident_chain);
 }
 
-// vec: the normalisation's 16-byte order (launch_normalize).
+// Whether that kernel normalises by itself (it sums in chunks of 4096 elements; only
+// batches of 65536 matrices and more are summed in larger ones).
+bool resident_normalizes(const Plan &p, int64_t batch) {
+    return muon_polar::norm_chunk(batch, p.m * p.n) == 4096;
+}
+
+// `steps` >= 1 steps in launches of up to kResidentSteps, the second and later ones in
+// place (a workgroup holds its whole matrix in LDS before it writes any of it), as the
+// first may be too.  vec: the normalisation's 16-byte order (launch_normalize).
 int run_resident(const Plan &p, const void *x, void *y, int64_t batch, const double *coefficients,
                  int64_t steps, bool normalize, bool vec, hipStream_t stream) {
-    muon_polar::ResidentArgs g{};
-    g.x = static_cast<const uint16_t *>(x);
-    g.y = static_cast<uint16_t *>(y);
-    g.m = static_cast<int32_t>(p.m);
-    g.n = static_cast<int32_t>(p.n);
-    g.tall = p.tall ? 1 : 0;
-    g.steps = static_cast<int32_t>(steps);
-    g.normalize = normalize ? 1 : 0;
-    g.vec = vec ? 1 : 0;
-    g.chunks = normalize ? static_cast<int32_t>(muon_polar::norm_chunks(batch, p.m * p.n)) : 0;
-    for (int64_t i = 0; i < 3 * steps; ++i) g.coef[i] = static_cast<float>(coefficients[i]);
-    return finish_stage(muon_polar::launch_resident(g, batch, stream), stream, "resident");
+    for (int64_t i = 0; i < steps; i += muon_polar::kResidentSteps) {
+        const int64_t count = std::min<int64_t>(steps - i, muon_polar::kResidentSteps);
+        const bool norm = normalize && i == 0;
+        muon_polar::ResidentArgs g{};
+        g.x = static_cast<const uint16_t *>(i == 0 ? x : y);
+        g.y = static_cast<uint16_t *>(y);
+        g.m = static_cast<int32_t>(p.m);
+        g.n = static_cast<int32_t>(p.n);
+        g.tall = p.tall ? 1 : 0;
+        g.steps = static_cast<int32_t>(count);
+        g.normalize = norm ? 1 : 0;
+        g.vec = vec ? 1 : 0;
+        g.chunks = norm ? static_cast<int32_t>(muon_polar::norm_chunks(batch, p.m * p.n)) : 0;
+        for (int64_t c = 0; c < 3 * count; ++c)
+            g.coef[c] = static_cast<float>(coefficients[3 * i + c]);
+        const int st = finish_stage(muon_polar::launch_resident(g, batch, stream), stream, "resident");
+        if (st != MUON_POLAR_OK) return st;
+    }
+    return MUON_POLAR_OK;
 }
 
 // One step given the workspace: left form (m <= n) or right-Gram form; rows the
@@ -1199,7 +1212,7 @@ int run_resident(const Plan &p, const void *x, void *y, int64_t batch, const dou
 int run_step(const Plan &p, const void *x, void *y, void *workspace, int64_t batch, double a,
              double b, double c, hipStream_t stream, int64_t ldx_in = 0, int64_t n_out = 0,
              bool force_pad = false) {
-    if (p.resident && ldx_in == 0 && n_out == 0) {
+    if (p.resident) {  // (single steps only: a resident plan's chains do not come here)
         const double coef[3] = {a, b, c};
         return run_resident(p, x, y, batch, coef, 1, false, false, stream);
     }
@@ -1334,10 +1347,12 @@ int update_tensors(const muon_polar::MuonTensors &t, void *workspace, size_t wor
     // The normalised input goes where the iterate chain starts (out for an even
     // step count, else scratch); the momentum pass writes the other buffer, which
     // the first step overwrites only after the normalisation has read it.
-    // (The resident kernel normalises by itself, from the scratch buffer.)
-    const bool resident = resident_runs(p, batch, steps, true);
+    // (The resident kernel normalises by itself, from the scratch buffer, and runs in
+    // place where the normalised input is out.)
+    const bool resident = resident_runs(p, steps, true);
+    const bool norm_inside = resident && resident_normalizes(p, batch);
     uint16_t *first = steps % 2 == 0 ? out : scratch;
-    uint16_t *x0 = steps % 2 == 0 || resident ? scratch : out;
+    uint16_t *x0 = steps % 2 == 0 || norm_inside ? scratch : out;
     const int64_t mn = m * n;
     st = finish_stage(
         muon_polar::launch_muon_momentum(t, x0, partial, mn, static_cast<float>(1.0 - momentum),
@@ -1345,15 +1360,15 @@ int update_tensors(const muon_polar::MuonTensors &t, void *workspace, size_t wor
                                          mn % 8 == 0 && vec_gb, stream),
         stream, "momentum");
     if (st != MUON_POLAR_OK) return st;
-    if (resident) {
-        st = run_resident(p, x0, out, batch, coefficients, steps, true, mn % 8 == 0, stream);
-    } else {
+    if (!norm_inside) {
         st = finish_stage(muon_polar::launch_norm_scale(x0, first, partial, batch, mn, mn % 8 == 0,
                                                         stream),
                           stream, "normalize");
         if (st != MUON_POLAR_OK) return st;
-        st = run_steps(p, workspace, first, out, scratch, batch, coefficients, steps, stream);
     }
+    st = resident ? run_resident(p, norm_inside ? x0 : first, out, batch, coefficients, steps,
+                                 norm_inside, mn % 8 == 0, stream)
+                  : run_steps(p, workspace, first, out, scratch, batch, coefficients, steps, stream);
     if (st != MUON_POLAR_OK) return st;
     return finish_stage(
         muon_polar::launch_muon_param_update(t, out, mn, static_cast<float>(1.0 - lr * weight_decay),
@@ -1777,15 +1792,17 @@ int muon_polar_express(const void *x, void *y, void *workspace, size_t workspace
 
     const uint16_t *cur = static_cast<const uint16_t *>(x);
     const bool vec = (m * n) % 8 == 0 && aligned16(x) && aligned16(iterate(0));
-    if (resident_runs(p, batch, steps, normalize != 0))
-        return run_resident(p, x, y, batch, coefficients, steps, normalize != 0, vec, stream);
-    if (normalize) {
+    const bool resident = resident_runs(p, steps, normalize != 0);
+    const bool norm_inside = resident && normalize && resident_normalizes(p, batch);
+    if (normalize && !norm_inside) {
         uint16_t *dst = iterate(0);
         st = finish_stage(muon_polar::launch_normalize(cur, dst, partial, batch, m * n, vec, stream),
                           stream, "normalize");
         if (st != MUON_POLAR_OK) return st;
         cur = dst;
     }
+    if (resident)
+        return run_resident(p, cur, out, batch, coefficients, steps, norm_inside, vec, stream);
     return run_steps(p, workspace, cur, out, scratch, batch, coefficients, steps, stream);
 }
 

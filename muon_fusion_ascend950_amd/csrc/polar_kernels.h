@@ -167,7 +167,7 @@ hipError_t launch_muon_param_update(const MuonTensors &t, const uint16_t *o, int
                                     float decay, float alpha, bool vec, hipStream_t stream);
 
 // Whole steps of small matrices, one workgroup each (polar_resident.hip).  x and y are
-// [batch, m, n] dense, any alignment; steps coefficient triples in coef; normalize: the
+// [batch, m, n] dense, any alignment, and may be the same; steps coefficient triples in coef; normalize: the
 // per-matrix normalisation first, in chunks of 4096 elements (norm_chunk must be 4096;
 // vec as launch_normalize's).
 constexpr int kResidentSteps = 8;

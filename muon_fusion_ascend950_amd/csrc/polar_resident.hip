@@ -8,7 +8,8 @@
 //
 // Sums run in the stage kernels' unsplit order (k ascending, one chain per output, a·X
 // added before the 64-element K-step that holds the output's rows), so the results are
-// theirs bit for bit; so is the normalisation's sum of squares.
+// theirs bit for bit; so is the normalisation's sum of squares.  Y may be X: a workgroup
+// has all of its matrix in LDS before it writes any of it.
 //
 // 16 waves.  Gram and poly: one 32x32 block of the upper triangle per wave at a time
 // (2x2 16x16x32 MFMAs).  Apply: wave w computes all its column blocks of row block

@@ -94,3 +94,21 @@ def test_a_chain_is_its_steps_where_only_the_chain_is_resident(monkeypatch, mf, 
     for c in O.COEFFICIENTS:
         want = mf.polar_step(want, *c)
     assert torch.equal(mf.polar_express(x, O.COEFFICIENTS, normalize=False), want)
+
+
+@pytest.mark.parametrize("steps", [8, 9, 16, 17])
+# the stages cut [2,31,1501]'s gram; tall; whole vectors; even
+@pytest.mark.parametrize("shape", [(2, 31, 1501), (3, 129, 257), (1, 257, 64), (2, 64, 96), (1, 95, 130)])
+def test_chains_of_any_length_are_their_steps(monkeypatch, mf, shape, steps):
+    for k in [k for k in os.environ if k.startswith("MUON_POLAR_") and k != "MUON_POLAR_CAPI_LIBRARY"]:
+        monkeypatch.delenv(k)
+    x = (O.make_input(shape, seed=65).float() * 11.0).to(torch.bfloat16).to(DEV)
+    coeffs = (O.COEFFICIENTS + O.COEFFICIENTS[4:] * 12)[:steps]
+    want = mf.polar_express(x, (), normalize=True)
+    for c in coeffs:
+        want = mf.polar_step(want, *c)
+    assert torch.isfinite(want).all() and torch.equal(mf.polar_express(x, coeffs), want)
+    from muon_fusion_ascend950_amd import capi
+
+    m, n = shape[1:] if shape[1] <= shape[2] or shape[2] % 8 == 0 else shape[:0:-1]
+    assert capi.check_plan(shape[0], m, n, cus=256, blocks_per_cu=(2, 2, 2)).resident == 3
