@@ -525,7 +525,7 @@ constexpr int64_t kMaxMatrixElems = int64_t(1) << 30;
 // same ([64,384,128] 56 / 97 us).  There the stages are neither split nor paired, so steps and
 // chains have the same bits on either route.
 bool resident_pays(int64_t batch, int64_t m, int64_t n, bool chain) {
-    if (muon_polar::resident_fit(m, n) == 0) return false;
+    if (!muon_polar::resident_fits(m, n)) return false;
     if (batch >= 256) return true;
     static constexpr int kBase[muon_polar::kResidentBlocks + 1] = {0, 150, 170, 320, 300, 410, 520};
     static constexpr int kSlope[muon_polar::kResidentBlocks + 1] = {0, 14, 26, 33, 54, 75, 110};

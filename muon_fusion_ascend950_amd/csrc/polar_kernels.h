@@ -178,8 +178,8 @@ struct ResidentArgs {
     int32_t m, n, tall, steps, normalize, vec, chunks;
     float coef[3 * kResidentSteps];
 };
-// KiB of LDS the kernel for [m, n] matrices uses (80 or 160), 0 when they do not fit.
-int resident_fit(int64_t m, int64_t n);
+// Whether [m, n] matrices fit the kernel.
+bool resident_fits(int64_t m, int64_t n);
 hipError_t launch_resident(const ResidentArgs &g, int64_t batch, hipStream_t stream);
 
 // Scratch of the allocation-free step (polar_noalloc.hip): a device array of

@@ -28,9 +28,10 @@ namespace {
 
 constexpr int kWaves = 16, kThreads = 64 * kWaves;
 constexpr int kRowPad = 8;         // elements
-constexpr int kColBlocks = 4;  // 32-column blocks of Y per wave, at most (resident_fit)
+constexpr int kColBlocks = 4;  // 32-column blocks of Y per wave, at most (resident_fits)
 constexpr int kMaxChunks = 64;     // partial sums of the normalisation
 constexpr int kTailBytes = 4 * (kMaxChunks + kWaves);
+constexpr int kLdsBytes = 160 * 1024;
 
 using lds_bf16x4 = __attribute__((address_space(3))) bf16x4;
 
@@ -41,10 +42,11 @@ __device__ __forceinline__ u32x4 rotate_words(u32x4 v, int k) {
     return v;
 }
 
-// NB: 32-row blocks of the shorter side.  LDS_KIB: static LDS (80: two workgroups per CU).
-template <int NB, int LDS_KIB>
+// NB: 32-row blocks of the shorter side.  All of the LDS, as one workgroup per CU runs
+// whatever it takes: 16 waves of over 64 registers (117 to 128) leave no room for another.
+template <int NB>
 __global__ __launch_bounds__(kThreads) void resident_kernel(ResidentArgs g) {
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[LDS_KIB * 1024];
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[kLdsBytes];
     constexpr int kSp = 32 * NB;
     const int tid = static_cast<int>(threadIdx.x);
     const int lane = tid & 63, l15 = lane & 15, lq = lane >> 4;
@@ -55,7 +57,7 @@ __global__ __launch_bounds__(kThreads) void resident_kernel(ResidentArgs g) {
     const int xs = 32 * lblocks + kRowPad, as = kSp + kRowPad;  // row strides in elements
     uint16_t *X = reinterpret_cast<uint16_t *>(smem);
     uint16_t *A = X + kSp * xs;
-    float *partial = reinterpret_cast<float *>(smem + LDS_KIB * 1024 - kTailBytes);
+    float *partial = reinterpret_cast<float *>(smem + kLdsBytes - kTailBytes);
     float *red = partial + kMaxChunks;
     const uint16_t *x = g.x + int64_t(blockIdx.x) * mn;
     uint16_t *y = g.y + int64_t(blockIdx.x) * mn;
@@ -428,36 +430,29 @@ __global__ __launch_bounds__(kThreads) void resident_kernel(ResidentArgs g) {
     }
 }
 
-template <int NB>
-const void *kernel_of(int kib) {
-    return kib == 80 ? reinterpret_cast<const void *>(&resident_kernel<NB, 80>)
-                     : reinterpret_cast<const void *>(&resident_kernel<NB, 160>);
-}
-
 }  // namespace
 
-int resident_fit(int64_t m, int64_t n) {
+bool resident_fits(int64_t m, int64_t n) {
     const int64_t s = m < n ? m : n, l = m < n ? n : m;
     const int64_t nb = (s + 31) / 32, lb = (l + 31) / 32;
-    if (nb > kResidentBlocks || lb > kColBlocks * (kWaves / nb)) return 0;
+    if (nb > kResidentBlocks || lb > kColBlocks * (kWaves / nb)) return false;
     const int64_t bytes =
         2 * 32 * nb * (32 * lb + kRowPad + 32 * nb + kRowPad) + kTailBytes;
-    return bytes <= 80 * 1024 ? 80 : bytes <= 160 * 1024 ? 160 : 0;
+    return bytes <= kLdsBytes;
 }
 
 hipError_t launch_resident(const ResidentArgs &g, int64_t batch, hipStream_t stream) {
-    const int kib = resident_fit(g.m, g.n);
-    if (kib == 0 || batch <= 0 || batch >= (int64_t(1) << 31) || g.steps < 0 ||
+    if (!resident_fits(g.m, g.n) || batch <= 0 || batch >= (int64_t(1) << 31) || g.steps < 0 ||
         g.steps > kResidentSteps || g.chunks > kMaxChunks)
         return hipErrorInvalidValue;
     const void *k = nullptr;
     switch (((g.m < g.n ? g.m : g.n) + 31) / 32) {
-        case 1: k = kernel_of<1>(kib); break;
-        case 2: k = kernel_of<2>(kib); break;
-        case 3: k = kernel_of<3>(kib); break;
-        case 4: k = kernel_of<4>(kib); break;
-        case 5: k = kernel_of<5>(kib); break;
-        case 6: k = kernel_of<6>(kib); break;
+        case 1: k = reinterpret_cast<const void *>(&resident_kernel<1>); break;
+        case 2: k = reinterpret_cast<const void *>(&resident_kernel<2>); break;
+        case 3: k = reinterpret_cast<const void *>(&resident_kernel<3>); break;
+        case 4: k = reinterpret_cast<const void *>(&resident_kernel<4>); break;
+        case 5: k = reinterpret_cast<const void *>(&resident_kernel<5>); break;
+        case 6: k = reinterpret_cast<const void *>(&resident_kernel<6>); break;
         default: return hipErrorInvalidValue;
     }
     ResidentArgs copy = g;
