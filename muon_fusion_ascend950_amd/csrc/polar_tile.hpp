@@ -66,10 +66,6 @@ __device__ __forceinline__ int kc_offset(int row, int chunk) {
 // constant offsets.
 __device__ __forceinline__ int kc_swz16(int row) { return (row >> 1) & 7; }
 
-__device__ __forceinline__ int kc_offset16(int row, int chunk) {
-    return row * kBK + ((chunk ^ kc_swz16(row)) << 3);
-}
-
 // N-contiguous tile [64][BN] (stage-3 X panel, rows = K): chunk c of K-row k is
 // stored at c ^ nc_swz(k).  A transposing read fetches 4 consecutive K-rows by
 // 2 chunks (32 B) per 16-lane group, and a half-wave (two groups: 16 adjacent
@@ -103,10 +99,6 @@ __device__ __forceinline__ int nc_swz16(int krow) {
     const int hi = ((krow >> 3) & 1) << 1;
     if constexpr (BN == 192) return (((krow >> 1) & 1) << 2) | hi;
     return ((krow & 3) << 2) | hi;
-}
-template <int BN>
-__device__ __forceinline__ int nc_offset16(int krow, int chunk) {
-    return krow * BN + ((chunk ^ nc_swz16<BN>(krow)) << 3);
 }
 
 // ---------------------------------------------------------------------------
