@@ -25,8 +25,20 @@ SHAPES = [(1, 1, 1), (3, 3, 5), (2, 7, 7), (1, 16, 17), (2, 31, 33), (1, 32, 204
 def mf(monkeypatch):
     import muon_fusion_ascend950_amd as module
 
-    monkeypatch.delenv("MUON_POLAR_RESIDENT", raising=False)
+    # (any variable that tunes the stages turns the resident kernel off)
+    for k in [k for k in os.environ if k.startswith("MUON_POLAR_") and k != "MUON_POLAR_CAPI_LIBRARY"]:
+        monkeypatch.delenv(k)
     return module
+
+
+def route(shape):
+    """1: single steps resident, 2: chains (tall odd widths run transposed)."""
+    from muon_fusion_ascend950_amd import capi
+
+    batch, m, n = shape
+    if m > n and n % 8:
+        m, n = n, m
+    return capi.check_plan(batch, m, n, cus=256, blocks_per_cu=(2, 2, 2)).resident
 
 
 def _stages(monkeypatch, f):
@@ -47,10 +59,12 @@ def test_steps_and_chains_have_the_stage_kernels_bits(monkeypatch, mf, shape):
              lambda: mf.polar_express(raw),
              lambda: mf.polar_express(x, O.COEFFICIENTS[:2], normalize=False),
              # more steps than one launch takes
-             lambda: mf.polar_express(raw, (O.COEFFICIENTS * 2)[:9])]
+             lambda: mf.polar_express(raw, O.COEFFICIENTS + O.COEFFICIENTS[4:] * 4)]
+    assert route(shape) == 3
     for f in calls:
         y = f()
         torch.cuda.synchronize()
+        assert torch.isfinite(y).all()
         want = _stages(monkeypatch, f)
         assert torch.equal(y.view(torch.int16), want.view(torch.int16))
 
@@ -86,9 +100,8 @@ def test_infinities_and_nans_stay_in_their_matrix(mf):
 
 
 @pytest.mark.parametrize("shape", [(64, 384, 128), (85, 352, 120)])
-def test_a_chain_is_its_steps_where_only_the_chain_is_resident(monkeypatch, mf, shape):
-    for k in [k for k in os.environ if k.startswith("MUON_POLAR_") and k != "MUON_POLAR_CAPI_LIBRARY"]:
-        monkeypatch.delenv(k)
+def test_a_chain_is_its_steps_where_only_the_chain_is_resident(mf, shape):
+    assert route(shape) == 2
     x = O.make_input(shape, seed=64).to(DEV)
     want = x
     for c in O.COEFFICIENTS:
@@ -99,16 +112,28 @@ def test_a_chain_is_its_steps_where_only_the_chain_is_resident(monkeypatch, mf, 
 @pytest.mark.parametrize("steps", [8, 9, 16, 17])
 # the stages cut [2,31,1501]'s gram; tall; whole vectors; even
 @pytest.mark.parametrize("shape", [(2, 31, 1501), (3, 129, 257), (1, 257, 64), (2, 64, 96), (1, 95, 130)])
-def test_chains_of_any_length_are_their_steps(monkeypatch, mf, shape, steps):
-    for k in [k for k in os.environ if k.startswith("MUON_POLAR_") and k != "MUON_POLAR_CAPI_LIBRARY"]:
-        monkeypatch.delenv(k)
+def test_chains_of_any_length_are_their_steps(mf, shape, steps):
+    assert route(shape) == 3
     x = (O.make_input(shape, seed=65).float() * 11.0).to(torch.bfloat16).to(DEV)
     coeffs = (O.COEFFICIENTS + O.COEFFICIENTS[4:] * 12)[:steps]
     want = mf.polar_express(x, (), normalize=True)
     for c in coeffs:
         want = mf.polar_step(want, *c)
     assert torch.isfinite(want).all() and torch.equal(mf.polar_express(x, coeffs), want)
-    from muon_fusion_ascend950_amd import capi
 
-    m, n = shape[1:] if shape[1] <= shape[2] or shape[2] % 8 == 0 else shape[:0:-1]
-    assert capi.check_plan(shape[0], m, n, cus=256, blocks_per_cu=(2, 2, 2)).resident == 3
+
+@pytest.mark.parametrize("steps", [1, 4, 5, 9])
+@pytest.mark.parametrize("shape", [(3, 40, 64), (2, 33, 130), (1, 31, 57), (2, 72, 40), (2, 57, 31)])
+def test_muon_updates_have_the_stage_kernels_bits(monkeypatch, mf, shape, steps):
+    assert route(shape) & 2
+    gen = torch.Generator(device=DEV).manual_seed(66)
+    p, g, b = (torch.randn(shape, generator=gen, device=DEV) for _ in range(3))
+    coeffs = O.COEFFICIENTS + O.COEFFICIENTS[4:] * 4
+
+    def update():
+        q, buf = p.clone(), b.clone()
+        mf.muon_update(q, g, buf, lr=0.1, ns_steps=steps, coefficients=coeffs)
+        return torch.stack([q, buf])
+
+    y = update()
+    assert torch.isfinite(y).all() and torch.equal(y, _stages(monkeypatch, update))
