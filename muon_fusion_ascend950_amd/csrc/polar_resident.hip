@@ -8,7 +8,9 @@
 //
 // Sums run in the stage kernels' unsplit order (k ascending, one chain per output, a·X
 // added before the 64-element K-step that holds the output's rows), so the results are
-// theirs bit for bit; so is the normalisation's sum of squares.  Y may be X: a workgroup
+// theirs bit for bit (but for shorter sides of 32, 96 or 160, which have no padded rows here:
+// infinities in X or A stay infinite where the stages' 64-row tiles make NaN of 0 * inf); so
+// is the normalisation's sum of squares.  Y may be X: a workgroup
 // has all of its matrix in LDS before it writes any of it.
 //
 // 16 waves.  Gram and poly: one 32x32 block of the upper triangle per wave at a time

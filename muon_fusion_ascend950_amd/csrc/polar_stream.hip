@@ -1,15 +1,16 @@
 // polar_stream.hip — DMA-fed variant of the three stage kernels.
 //
-// Same tiles, MFMA layout and arithmetic as the register-staged kernels in
-// polar_kernels.hip; what changes is how data moves:
+// Same tiles and arithmetic as the register-staged kernels in polar_kernels.hip (the large
+// tiles on 16x16x32 MFMAs, whose results have the same bits); what changes is how data moves:
 //
 //   * global -> LDS by buffer_load_dwordx4 ... lds (no VGPR staging, no
 //     ds_write), 1 KiB per wave instruction, swizzle applied on the global side;
-//   * an LDS ring of D K-step slots (2 for 256x256 tiles; up to 8 for the
-//     latency-bound small tiles): panels k+1 .. k+D-1 stream in while step k is
-//     multiplied; one barrier per K-step, placed so that the MFMA pipe keeps a
-//     k16 slice of work queued across it, and the DMA instructions of the next
-//     panel are interleaved one by one with that slice's MFMAs;
+//   * an LDS ring: D K-step slots, up to 8 for the latency-bound small tiles, or, for
+//     256x256 and 128x128 tiles with 8 waves, five or nine row and column panels in turn
+//     (StreamGeom): later panels stream in while step k is multiplied; one barrier per
+//     K-step, placed so that the MFMA pipe keeps a slice of work queued across it, and
+//     the DMA instructions of the next panels are interleaved one by one with MFMAs (the
+//     panel rings: spread evenly over the whole step);
 //   * MFMA operand fragments double-buffered in registers: the LDS reads of
 //     slice s+1 are in flight while slice s is multiplied (with one MFMA per
 //     slice, 64x64 tiles, a whole K-step's reads run one step ahead instead);
@@ -46,10 +47,9 @@ namespace {
 // wave tiles: 1.5x the fragment reads, but one wave's LDS and barrier waits are
 // covered by the other's MFMAs).  D = ring depth (LDS slots of one K-step each):
 // panels k+1 .. k+D-1 are in flight while step k is multiplied.  Two slots suit
-// the MFMA-bound shapes (a third measured slower at 4096 x 14336: more DMA in
-// flight competes with the fragment reads); deeper rings serve latency-bound
-// launches with few K-steps per workgroup, where each step would otherwise wait
-// for one full memory round trip.
+// the MFMA-bound shapes; deeper rings serve latency-bound launches with few K-steps per
+// workgroup, where each step would otherwise wait for one full memory round trip.  Panel
+// rings (kPanelRing below) take D = 2 for five panels, D = 4 for nine.
 template <int BM, int BN, int NW, int D, int KT = 0>
 struct StreamGeom {
     static constexpr int kThreads = 64 * NW;
@@ -171,13 +171,14 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
     constexpr int WM = BM / 2, WN = DG ? BN : BN / (kGridWaves / 2);
     constexpr bool kPanelRing = Geo::kPanelRing;
     constexpr int kPanels = Geo::kPanels;
-    // MFMA shape: 16x16x32 in the large-tile kernels (256x256 with 8 waves, the wave
-    // pairs), else 32x32x16.  The large tiles run at the power limit (the clock falls as
+    // MFMA shape: 16x16x32 in the panel rings (256x256 and 128x128 with 8 waves) and the
+    // wave pairs, else 32x32x16.  The large tiles run at the power limit (the clock falls as
     // the MFMA pipe fills), and 16x16x32 takes less power per FLOP: a loop of MFMAs alone
-    // on random operands sustains 2069 against 1819 TFLOP/s, with the fragment reads of
-    // 128x64 wave tiles 1739 against 1617.  Same bits (mfma_16x16x32).  With the even DMA
-    // spacing below: [4096,14336] gram 207.7 -> 185.1 us, poly 72.0 -> 65.6, apply 393.1
-    // -> 351.3; [4,4096,4096] 257.8 -> 233.9, 266.8 -> 241.7, 451.3 -> 409.2.
+    // on random operands sustains 2043 against 1817 TFLOP/s, with the fragment reads of
+    // 128x64 wave tiles 1786 against 1624 (one box; 2069 and 1819 on another).  Same bits
+    // (mfma_16x16x32).  With the even DMA spacing below: [4096,14336] gram 207.7 -> 185.1
+    // us, poly 72.0 -> 65.6, apply 393.1 -> 351.3; [4,4096,4096] 257.8 -> 233.9, 266.8 ->
+    // 241.7, 451.3 -> 409.2.
     // kB: the MFMA's rows and columns; kNQ: groups of 4 consecutive columns a lane holds
     // of one block.
     constexpr bool k16 = kPair || kPanelRing;
@@ -696,8 +697,8 @@ __device__ __forceinline__ void stream_segment(const GemmArgs &g, uint16_t *smem
         // DMA instruction every kGap MFMAs over slice s1 and the next step's s0.  Issued
         // together behind the barrier, a step's instructions (256x256: 64 of 16 clocks
         // each in the CU's address unit, half of the step's MFMA time) queue up and hold
-        // the waves' MFMAs back: MFMA pipe busy 68% of apply's cycles at [4096,14336] with
-        // two 64 KiB slots, 78% spread.  The half step that five panels hold beyond two
+        // the waves' MFMAs back: MFMA pipe busy 64% of apply's cycles at [4096,14336] with
+        // two 64 KiB slots, 67% spread (62 and 66% at [4,4096,4096]).  The half step that five panels hold beyond two
         // slots gives them time to land (8 MFMAs apart: 351 us; 4: 359).  128x128 tiles,
         // five panels against two slots: [8,512,2048] apply 14.7 -> 13.3 us, [1,2560,4096]
         // apply 68.6 -> 58.6, [32,1024,1024] step 173.7 -> 157.5; nine against four slots:
@@ -1414,10 +1415,11 @@ __global__ __launch_bounds__(512) void polar_stream_halves_kernel(GemmArgs g) {
     }
 }
 
-// Instantiated (tile, waves, depth) combinations: 256x256 with 8 or 4 waves and
-// two slots; 128x128 with 8 or 4 waves and 2 or 4 slots of 32 KiB (8 waves: two
-// per SIMD, 64x32 wave tiles; [16,512,2048] 62.5 -> 59.0 us, [1,1024,4096]
-// 46.3 -> 43.9 us against 4 waves); 192x192 with 8 waves (the wave pairs) and 2
+// Instantiated (tile, waves, depth) combinations: 256x256 with 8 waves (five panels of
+// 32 KiB, depth 2) or 4 waves and two slots; 128x128 with 8 waves (two per SIMD, 64x32
+// wave tiles; five or nine panels of 16 KiB, depth 2 or 4, or two slots where rows
+// straddle cache lines; [16,512,2048] 62.5 -> 59.0 us, [1,1024,4096] 46.3 -> 43.9 us
+// against 4 waves) or with 4 waves and 2 or 4 slots of 32 KiB; 192x192 with 8 waves (the wave pairs) and 2
 // or 3 slots of 48 KiB (three by default: [4096,14336] gram 225 -> 212 us, poly
 // 75 -> 72 us), or with 4 waves and 2 slots; other tiles with 4 waves and the
 // depths their LDS allows (64x64: 2, 4 or 8 of 16 KiB; 128x256 and 256x128: 2 or 3
