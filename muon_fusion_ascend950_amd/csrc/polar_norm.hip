@@ -179,24 +179,38 @@ __device__ __forceinline__ float lerp_rounded(float start, float end, float w) {
     return fabsf(w) < 0.5f ? start + w * (end - start) : end - (end - start) * (1.0f - w);
 }
 
-// Where tensor t of the Muon update's fp32 tensors (and of its gradient, G = float or
-// the bits of a bf16) lies: one batched tensor, or tensors of their own, whose pointers
-// travel in the kernel arguments (no table in memory to fill and to wait for).  One
-// pointer per tensor, however many matrices it holds: one per matrix took a launch for
-// every 128 of them: the update of 4 x [4096,32,32] 1073 us, now 671.
+// Where matrix b of the Muon update's fp32 tensors (and of its gradient, G = float or
+// the bits of a bf16) lies: rows of one batched tensor, or tensors of their own, whose
+// pointers travel in the kernel arguments (no table in memory to fill and to wait for):
+// one matrix in each (the common case: 8 x [768,768] 13.0 us a launch, 13.6 with a branch
+// around the division), or `per` of them.  One pointer per matrix took a launch for every 128 of them: the update
+// of 4 x [4096,32,32] 1073 us, now 671.
 template <typename G>
 struct BatchedMats {
     const G *g;
     float *w;
-    __device__ __forceinline__ const G *grad(int) const { return g; }
-    __device__ __forceinline__ float *buf(int) const { return w; }
+    int64_t mn;
+    __device__ __forceinline__ const G *grad(int b) const { return g + int64_t(b) * mn; }
+    __device__ __forceinline__ float *buf(int b) const { return w + int64_t(b) * mn; }
 };
 template <typename G>
 struct ListedMats {
     const G *g[kMuonListMax];
     float *w[kMuonListMax];
-    __device__ __forceinline__ const G *grad(int t) const { return g[t]; }
-    __device__ __forceinline__ float *buf(int t) const { return w[t]; }
+    __device__ __forceinline__ const G *grad(int b) const { return g[b]; }
+    __device__ __forceinline__ float *buf(int b) const { return w[b]; }
+};
+template <typename G>
+struct ListedTensors {
+    ListedMats<G> t;
+    int64_t mn;
+    int32_t per;
+    __device__ __forceinline__ const G *grad(int b) const {
+        return t.g[b / per] + int64_t(b % per) * mn;
+    }
+    __device__ __forceinline__ float *buf(int b) const {
+        return t.w[b / per] + int64_t(b % per) * mn;
+    }
 };
 struct BatchedParam {
     float *p;
@@ -240,8 +254,8 @@ __device__ __forceinline__ void load8(const uint16_t *g, float (&v)[8]) {
 __device__ __forceinline__ float grad_value(float g) { return g; }
 __device__ __forceinline__ float grad_value(uint16_t g) { return bf16_bits_to_f32(g); }
 
-// Momentum pass of the Muon update over chunk c of matrix b of tensor blockIdx.y, which
-// holds `per` of them (chunks as in norm_partial_kernel):
+// Momentum pass of the Muon update over chunk c of matrix b (chunks as in
+// norm_partial_kernel):
 //     buf ← lerp(buf, g, w)                  (w = 1 − momentum)
 //     g'  = lerp(g, buf, momentum) | buf     (Nesterov or plain)
 //     x0  = bf16(g'),   partial[b, c] = Σ x0²  in norm_partial_kernel's order
@@ -257,13 +271,13 @@ __device__ __forceinline__ float grad_value(uint16_t g) { return bf16_bits_to_f3
 template <bool kOrder8, bool kVec, typename G, typename Mats>
 __global__ __launch_bounds__(kNormThreads) void muon_momentum_kernel(
     const Mats mats, uint16_t *__restrict__ x0, float *__restrict__ partial, int64_t mn,
-    int per, int chunks, int64_t chunk, float w, float beta, int nesterov) {
+    int chunks, int64_t chunk, float w, float beta, int nesterov) {
 #pragma clang fp contract(off)
     __shared__ float red[4];
     const int b = blockIdx.x / chunks, c = blockIdx.x - b * chunks;
-    const int64_t base = (int64_t(blockIdx.y) * per + b) * mn;
-    const G *__restrict__ gb = mats.grad(blockIdx.y) + int64_t(b) * mn;
-    float *__restrict__ bufb = mats.buf(blockIdx.y) + int64_t(b) * mn;
+    const int64_t base = int64_t(b) * mn;
+    const G *__restrict__ gb = mats.grad(b);
+    float *__restrict__ bufb = mats.buf(b);
     const int64_t e0 = int64_t(c) * chunk;
     const int64_t e1 = e0 + chunk < mn ? e0 + chunk : mn;
     float acc = 0.0f;
@@ -332,7 +346,7 @@ __global__ __launch_bounds__(kNormThreads) void muon_momentum_kernel(
         }
     }
     const float t = block_sum(acc, red);
-    if (threadIdx.x == 0) partial[int64_t(blockIdx.y) * gridDim.x + blockIdx.x] = t;
+    if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
 // p ← p·decay + alpha·O over `total` elements of tensor blockIdx.y (fp32 p, bf16 O;
@@ -481,21 +495,20 @@ hipError_t launch_norm_scale(const uint16_t *x, uint16_t *y, const float *partia
 namespace {
 
 template <typename G, typename Mats>
-hipError_t launch_momentum_pass(const Mats &mats, uint16_t *x0, float *partial, int64_t tensors,
-                                int64_t matrices, int64_t mn, int64_t chunk, float w, float beta,
-                                bool nesterov, bool vec, hipStream_t stream) {
+hipError_t launch_momentum_pass(const Mats &mats, uint16_t *x0, float *partial, int64_t matrices,
+                                int64_t mn, int64_t chunk, float w, float beta, bool nesterov,
+                                bool vec, hipStream_t stream) {
     const int64_t chunks = (mn + chunk - 1) / chunk;
     const int64_t grid = matrices * chunks;
-    if (grid <= 0 || grid * tensors >= (int64_t(1) << 31)) return hipErrorInvalidValue;
+    if (grid <= 0 || grid >= (int64_t(1) << 31)) return hipErrorInvalidValue;
     const void *fn =
         mn % 8 != 0 ? reinterpret_cast<const void *>(&muon_momentum_kernel<false, false, G, Mats>)
         : vec       ? reinterpret_cast<const void *>(&muon_momentum_kernel<true, true, G, Mats>)
                     : reinterpret_cast<const void *>(&muon_momentum_kernel<true, false, G, Mats>);
-    int per = static_cast<int>(matrices), ch = static_cast<int>(chunks), nv = nesterov ? 1 : 0;
-    void *args[] = {const_cast<Mats *>(&mats), &x0, &partial, &mn, &per, &ch, &chunk, &w, &beta,
-                    &nv};
-    return hipLaunchKernel(fn, dim3(static_cast<unsigned>(grid), static_cast<unsigned>(tensors)),
-                           dim3(kNormThreads), args, 0, stream);
+    int ch = static_cast<int>(chunks), nv = nesterov ? 1 : 0;
+    void *args[] = {const_cast<Mats *>(&mats), &x0, &partial, &mn, &ch, &chunk, &w, &beta, &nv};
+    return hipLaunchKernel(fn, dim3(static_cast<unsigned>(grid)), dim3(kNormThreads), args, 0,
+                           stream);
 }
 
 template <typename G>
@@ -503,22 +516,27 @@ hipError_t momentum_of(const MuonTensors &t, uint16_t *x0, float *partial, int64
                        float beta, bool nesterov, bool vec, hipStream_t stream) {
     const int64_t chunk = norm_chunk(t.count * t.matrices, mn);
     if (t.count == 1) {
-        const BatchedMats<G> mats{static_cast<const G *>(t.grad[0]), static_cast<float *>(t.buf[0])};
-        return launch_momentum_pass<G>(mats, x0, partial, 1, t.matrices, mn, chunk, w, beta,
-                                       nesterov, vec, stream);
+        const BatchedMats<G> mats{static_cast<const G *>(t.grad[0]), static_cast<float *>(t.buf[0]),
+                                  mn};
+        return launch_momentum_pass<G>(mats, x0, partial, t.matrices, mn, chunk, w, beta, nesterov,
+                                       vec, stream);
     }
     for (int64_t i0 = 0; i0 < t.count; i0 += kMuonListMax) {
         const int64_t cnt = t.count - i0 < kMuonListMax ? t.count - i0 : kMuonListMax;
-        ListedMats<G> mats{};
+        ListedTensors<G> mats{{}, mn, static_cast<int32_t>(t.matrices)};
         for (int64_t i = 0; i < cnt; ++i) {
-            mats.g[i] = static_cast<const G *>(t.grad[i0 + i]);
-            mats.w[i] = static_cast<float *>(t.buf[i0 + i]);
+            mats.t.g[i] = static_cast<const G *>(t.grad[i0 + i]);
+            mats.t.w[i] = static_cast<float *>(t.buf[i0 + i]);
         }
         const int64_t m0 = i0 * t.matrices;
-        hipError_t e = launch_momentum_pass<G>(mats, x0 + m0 * mn,
-                                               partial + m0 * ((mn + chunk - 1) / chunk), cnt,
-                                               t.matrices, mn, chunk, w, beta, nesterov, vec,
-                                               stream);
+        uint16_t *xi = x0 + m0 * mn;
+        float *pi = partial + m0 * ((mn + chunk - 1) / chunk);
+        const hipError_t e =
+            t.matrices == 1
+                ? launch_momentum_pass<G>(mats.t, xi, pi, cnt, mn, chunk, w, beta, nesterov, vec,
+                                          stream)
+                : launch_momentum_pass<G>(mats, xi, pi, cnt * t.matrices, mn, chunk, w, beta,
+                                          nesterov, vec, stream);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
